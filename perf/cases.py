@@ -85,8 +85,10 @@ def draw(rng):
     if fam == "mx":
         fmt = rng.choice(["e4m3", "e5m2", "e2m1"])
         return dict(fam=fam, m=m, n=n, k=256 * rng.randint(4, 16), fmt=fmt)
-    layout = rng.choice(["nk", "nk", "kn"])
-    return dict(fam=fam, m=m, n=n, k=k, layout=layout, rt=rng.choice(["static", "runtime"]))
+    layout, rt = rng.choice(["nk", "nk", "kn"]), rng.choice(["static", "runtime"])
+    if layout == "kn" and rt == "runtime":
+        k = (k + 127) // 128 * 128
+    return dict(fam=fam, m=m, n=n, k=k, layout=layout, rt=rt)
 
 
 def _group(case, build, rows):
