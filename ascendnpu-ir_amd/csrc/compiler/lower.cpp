@@ -2401,6 +2401,67 @@ void hivmMatmulEpilogue(const Op *mm, bool intAcc, std::ostringstream &epi, std:
 }
 
 constexpr int MK_BF16_CODE = 1; // hf::MK_BF16
+
+// The tile of a contraction.  A tile's time is what its CU takes to pull
+// (tm + tn) K bytes through its LDS and multiply them, and 256 CUs work at
+// once: large tiles move fewer bytes, small ones fill the chip.  The times
+// below are measured (us per 4096 bytes of K beyond an empty launch's 2.3 us,
+// W8A8 and bf16 alike at N = 4096): `one` workgroup on a CU, a `second` beside
+// it, each one `more` (0: a CU holds one, the next wait).  Both sides of the
+// lines they draw, W8A8 at N = K = 4096: M = 64: 6.1 us (32x32) against 10.1
+// (64x64); M = 128: 8.5 (64x32) against 10.7 (64x64); M = 333: 12.8 (64x64)
+// against 13.5 (128x64); M = 1024: 22.6 (128x128) against 23.8 (128x64) and
+// 31.6 (256x128); M = 2048: 40.7 (256x128) against 46.1 (128x128 and
+// 256x256); block-scaled fp8, M = 2048: 56.6 (256x256) against 60.9 (128x128).
+struct ContractionTile {
+  char kind;           // 's' mmad_skinny, 't' mmad_tile, 'r' the 256x256 ring kernels of hf_mmad.h
+  int tm, tn, a, b, s; // 's': a waves; 't': a x b waves, s ring stages
+  double one, second, more;
+  bool operator==(const ContractionTile &o) const { return kind == o.kind && tm == o.tm && tn == o.tn; }
+  int threads() const { return kind == 'r' ? 512 : 64 * a * (kind == 's' ? 1 : b); }
+  // workgroups of one row of tiles (in eighths: an XCD each)
+  int64_t blocksPerRow(int64_t N) const {
+    const int64_t t = (N + tn - 1) / tn;
+    return kind == 'r' ? t : (t + 7) / 8 * 8;
+  }
+};
+const ContractionTile kRing256 = {'r', 256, 256, 0, 0, 0, 60, 0, 0};
+
+ContractionTile pickTile(int64_t M, int64_t N, int64_t Kb, bool bT, int mk) {
+  static const std::vector<ContractionTile> nk = {
+      {'s', 16, 16, 8, 0, 0, 2.4, 0, 0},   {'s', 32, 16, 8, 0, 0, 2.8, 0, 0},    {'s', 32, 32, 8, 0, 0, 3.8, 0, 0},
+      {'s', 64, 32, 4, 0, 0, 6.2, 0, 0},   {'t', 64, 64, 2, 2, 3, 8.4, 4, 7.5},  {'t', 128, 64, 4, 2, 3, 12, 10, 14},
+      {'t', 128, 128, 4, 4, 3, 20.5, 0, 0}, {'t', 256, 128, 4, 2, 3, 35, 0, 0},  kRing256};
+  // B [K, N]: short pieces of every k-row make the narrow tiles slower
+  static const std::vector<ContractionTile> kn = {
+      {'s', 16, 16, 8, 0, 0, 6.9, 0, 0},  {'s', 32, 16, 8, 0, 0, 7.4, 0, 0},       {'s', 32, 32, 8, 0, 0, 8.6, 0, 0},
+      {'t', 32, 64, 1, 2, 4, 9, 5, 6},    {'t', 64, 64, 2, 2, 3, 10.2, 6.5, 8}, {'t', 128, 64, 4, 2, 3, 12.6, 10, 14.5},
+      {'t', 128, 128, 4, 4, 3, 21, 0, 0}, {'t', 256, 128, 4, 2, 3, 36.5, 0, 0},  kRing256};
+  // block-scaled (the scaled instruction takes wider wave tiles)
+  static const std::vector<ContractionTile> fp8 = {
+      {'t', 32, 64, 1, 2, 4, 8, 0, 0}, {'t', 64, 64, 2, 2, 3, 12, 0, 0}, {'t', 64, 128, 2, 2, 3, 15.3, 0, 0},
+      {'t', 128, 128, 4, 2, 3, 28.5, 0, 0}, {'r', 256, 256, 0, 0, 0, 75, 0, 0}};
+  static const std::vector<ContractionTile> fp4 = {
+      {'t', 32, 64, 1, 2, 4, 9, 0, 0}, {'t', 64, 64, 2, 2, 3, 13, 0, 0}, {'t', 64, 128, 2, 4, 3, 19, 0, 0},
+      {'t', 128, 128, 4, 2, 3, 30, 0, 0}, {'r', 256, 256, 0, 0, 0, 102, 0, 0}};
+  const std::vector<ContractionTile> &cand = mk == 7 ? fp4 : mk >= 3 ? fp8 : bT ? nk : kn;
+  const ContractionTile *best = nullptr;
+  double bestCost = 0;
+  for (const ContractionTile &t : cand) {
+    // (the 256x256 ring of 64-byte slices took 650 us at M = 3000, N = 4096,
+    // K = 4032, where the 256x128 tiles take 76)
+    if (t.kind == 'r' && Kb % 128 != 0) continue;
+    const double n = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn) / 256;
+    double cost = n <= 1 ? t.one : !t.second ? t.one * std::ceil(n) : n <= 2 ? t.one + t.second * (n - 1) : t.one + t.second + t.more * (n - 2);
+    // the ring kernels leave the other CUs' power and L2 to the busy ones:
+    // with an eighth or a half of the CUs busy a tile takes 0.67 or 0.75 of
+    // its time with all of them
+    if (t.kind == 'r' && n < 1) cost *= 0.67 + 0.33 * n * n;
+    if (!best || cost < bestCost) { best = &t; bestCost = cost; }
+  }
+  return *best;
+}
+
 KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions &opt) {
   Func &f = *A.f;
   const Op *mm = findOp(f, [](const Op *o) {
@@ -2511,11 +2572,17 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
   // transposing reads).
   // An A [K, M] is staged and read the same way.
   const bool kmajOk = (bT || (N * esz) % 16 == 0) && (!aT || (M * esz) % 16 == 0);
-  const int dma = mx ? 4 : dma0 == 3 && (!bT || aT) && kmajOk ? 4 : dma0;
+  // smaller tiles where 256x256 ones would leave CUs idle (these take any K
+  // spanning a multiple of 64 bytes, and a B [K, N] as it is)
+  const bool tiles = !aT && dma0 != 0 && kmajOk && offs32 && !(mx && opt.mxExact);
+  // (a runtime row count: the tile for the largest; the others below)
+  const ContractionTile tile = tiles ? pickTile(M, N, K * esz, bT, mk) : kRing256;
+  const bool ring = tile.kind == 'r';
+  const int dma = !ring ? 0 : mx ? 4 : dma0 == 3 && (!bT || aT) && kmajOk ? 4 : dma0;
   const bool preB = dma != 0 && dma != 4 && !bT, preA = dma != 0 && dma != 4 && aT;
   const bool kT = (dma != 0 && dma != 4) || bT; // the main kernel's B is [N, K]
   const bool mT = (dma == 0 || dma == 4) && aT; // the main kernel's A is [K, M]
-  const int threads = dma >= 3 ? 512 : 256;
+  const int threads = !ring ? tile.threads() : dma >= 3 ? 512 : 256;
   auto align256 = [](uint64_t v) { return (v + 255) / 256 * 256; };
   const uint64_t wsB = preB ? align256((uint64_t)(N * K * esz)) : 0, wsA = preA ? align256((uint64_t)(M * K * esz)) : 0;
   // matmul_mx with mx_exact=1: both operands scaled into bf16 by pre kernels
@@ -2647,14 +2714,46 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
   for (size_t i = 0; i < A.params.size(); ++i)
     if (A.params[i].role == "scalar") k << "    const uint64_t s" << i << " = P.s" << i << ";\n";
   k << epi.str() << "    return (out_t)" << name[outv] << ";\n  }\n};\n}\n";
-  k << "extern \"C\" __global__ __launch_bounds__(" << threads << ") void " << kname << "(" << params << ") {\n"
-    << "  " << kname << "_args P;\n";
-  for (size_t i = 0; i < A.params.size(); ++i)
-    k << "  P." << (A.params[i].role == "scalar" ? "s" : "p") << i << " = " << (A.params[i].role == "scalar" ? "s" : "p") << i << ";\n";
+  auto kernelHead = [&](const std::string &name, int nthreads) {
+    k << "extern \"C\" __global__ __launch_bounds__(" << nthreads << ") void " << name << "(" << params << ") {\n"
+      << "  " << kname << "_args P;\n";
+    for (size_t i = 0; i < A.params.size(); ++i)
+      k << "  P." << (A.params[i].role == "scalar" ? "s" : "p") << i << " = " << (A.params[i].role == "scalar" ? "s" : "p") << i << ";\n";
+  };
   const std::string et = i8 ? "int8_t" : "uint16_t";
   const std::string aPtr = preA ? "(const " + et + "*)((char*)ws + " + std::to_string(wsB) + ")" : "(const " + et + "*)p" + std::to_string(a->argIdx);
   const std::string bPtr = preB ? "(const " + et + "*)ws" : "(const " + et + "*)p" + std::to_string(b->argIdx);
-  if (mxExact)
+  auto tileCall = [&](const ContractionTile &t) {
+    const std::string tt = mx ? "uint8_t" : et;
+    k << "  hf::" << (mx ? "mmad_mx<" : t.kind == 's' ? "mmad_skinny<" : "mmad_tile<") << mk << ", " << kname << "_epi, "
+      << (mx ? "" : bT ? "false, " : "true, ");
+    if (t.kind == 's') k << t.tm / 16 << ", " << t.tn / 16 << ", " << t.a;
+    else k << t.tm << ", " << t.tn << ", " << t.a << ", " << t.b << ", " << t.s;
+    k << ">((const " << tt << "*)p" << a->argIdx << ", (const " << tt << "*)p" << b->argIdx;
+    if (mx) k << ", (const uint8_t*)p" << sa->argIdx << ", (const uint8_t*)p" << sb->argIdx;
+    k << ", (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
+  };
+  // a runtime row count: the tile that each count would be given, up to the
+  // first that takes the main kernel's 256x256 ring
+  if (A.rowsDyn && tiles) {
+    std::vector<ContractionTile> emitted;
+    for (int64_t m = 16; m <= 16384; m += m < 64 ? 16 : 64) {
+      const ContractionTile t = pickTile(m, N, K * esz, bT, mk);
+      if (t.kind == 'r') break;
+      const std::string nm = kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn);
+      if (!p.alts.empty() && p.alts.back().name == nm) { p.alts.back().maxRows = m; continue; }
+      if (std::find(emitted.begin(), emitted.end(), t) == emitted.end()) {
+        emitted.push_back(t);
+        kernelHead(nm, t.threads());
+        tileCall(t);
+      }
+      p.alts.push_back({nm, m, t.tm, t.blocksPerRow(N), (unsigned)t.threads()});
+    }
+  }
+  kernelHead(kname, threads);
+  if (!ring)
+    tileCall(tile);
+  else if (mxExact)
     k << "  hf::mmad<" << MK_BF16_CODE << ", " << kname << "_epi, false, false, 4>((const uint16_t*)ws, (const uint16_t*)((char*)ws + "
       << wsXA << "), (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
   else if (mx)
@@ -2699,15 +2798,14 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
     p.workspaceBytes = wsXA + wsXB;
   }
   p.source = k.str();
-  // 256x256 macro-tiles, one workgroup each (XCD-aware order inside the kernel)
-  const int64_t TM = 256, TN = 256;
-  p.grid[0] = (unsigned)(((M + TM - 1) / TM) * ((N + TN - 1) / TN));
+  // macro-tiles, one workgroup each (XCD-aware order inside the kernel)
+  const int64_t TM = tile.tm, TN = tile.tn;
+  p.grid[0] = (unsigned)((M + TM - 1) / TM * tile.blocksPerRow(N));
   if (A.rowsDyn) {
-    // ceil(M / 256) row tiles of ceil(N / 256) tiles each
     p.rowsDyn = true;
     p.rowsA = 1;
     p.rowsB = TM;
-    p.rowsC = (N + TN - 1) / TN;
+    p.rowsC = tile.blocksPerRow(N);
   }
   p.block[0] = (unsigned)threads;
   static const char *mxName[5] = {"e4m3 x e4m3", "e4m3 x e5m2", "e5m2 x e4m3", "e5m2 x e5m2", "e2m1 x e2m1, fp4 two per byte"};
@@ -2719,7 +2817,8 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
               (preA || preB ? " (re-laid K-contiguous by a transpose kernel)" : "") +
               (dma == 4 ? std::string(", LDS DMA ring (128-byte slices, 2 waves/SIMD; ") + (aT && bT ? "A" : aT ? "A and B" : "B") +
                               " k-rows staged whole, transposing LDS reads)" :
-               dma == 3 ? ", LDS DMA ring (128-byte slices, 2 waves/SIMD)" : dma == 1 ? ", LDS DMA ring" : ", register staging");
+               dma == 3 ? ", LDS DMA ring (128-byte slices, 2 waves/SIMD)" : dma == 1 ? ", LDS DMA ring" : !ring ? ", LDS DMA ring, " + std::to_string(TM) + "x" + std::to_string(TN) + " tiles" + (tile.kind == 's' ? ", K split over the waves" : "") :
+               ", register staging");
   p.algoOps = 2.0 * (double)M * (double)N * (double)Kl;
   return p;
 }
@@ -4229,7 +4328,7 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
 std::string emitTranslationUnit(const std::vector<KernelPlan> &plans) {
   std::ostringstream s;
   s << "// Generated by bishengir-compile --target=mi355x (ConvertHFusionToHIP).\n"
-    << "#include \"hf_ops.h\"\n#include \"hf_row.h\"\n#include \"hf_argmax.h\"\n#include \"hf_mmad.h\"\n#include \"hf_misc.h\"\n"
+    << "#include \"hf_ops.h\"\n#include \"hf_row.h\"\n#include \"hf_argmax.h\"\n#include \"hf_mmad.h\"\n#include \"hf_mmsk.h\"\n#include \"hf_mmtl.h\"\n#include \"hf_misc.h\"\n"
     << "#include \"hf_rmsq.h\"\n#include \"hf_rmsn.h\"\n#include \"hf_sort.h\"\n\n";
   for (auto &p : plans) s << "// group @" << p.funcName << ": " << p.kind << " (" << p.variant << ")\n" << p.source << "\n";
   return s.str();
@@ -4264,6 +4363,8 @@ std::string emitManifest(const KernelPlan &p, const std::string &hsacoName) {
     for (auto &k : pk.kargs) s << " " << k;
     s << "\n";
   }
+  for (auto &a : p.alts)
+    s << "alt " << a.name << " " << a.maxRows << " " << a.rowsB << " " << a.rowsC << " " << a.block << "\n";
   s << "variant " << p.variant << "\n";
   return s.str();
 }

@@ -46,6 +46,15 @@ struct KernelPlan {
     std::vector<std::string> kargs;
   };
   std::vector<PreKernel> pre;
+  // other kernels of the group for small runtime row counts, by ascending
+  // maxRows: a launch of R <= maxRows rows runs the first that fits, without
+  // the pre kernels, on ceil(R / rowsB) * rowsC blocks, instead of the main one
+  struct RowAlt {
+    std::string name;
+    int64_t maxRows = 0, rowsB = 1, rowsC = 1;
+    unsigned block = 256;
+  };
+  std::vector<RowAlt> alts;
   // runtime row count (compiler option dyn=runtime): the kernel takes the
   // row count R as its last argument (karg "rows"); the launch grid is
   // min(ceil(R * rowsA / rowsB) * rowsC, rowsCap) blocks (rowsCap 0: no cap),

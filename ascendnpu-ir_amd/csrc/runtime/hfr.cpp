@@ -56,9 +56,19 @@ struct PreLaunch {
   std::vector<Karg> kargs;
 };
 
+// A kernel that takes the main kernel's place (without the pre kernels) for
+// launches of at most maxRows runtime rows: ceil(R / rowsB) * rowsC blocks.
+struct RowAlt {
+  std::string kernel;
+  hipFunction_t fn = nullptr;
+  int64_t maxRows = 0, rowsB = 1, rowsC = 1;
+  unsigned block = 0;
+};
+
 struct hfr_group {
   std::string func, kernel, hsaco;
   std::vector<PreLaunch> pre;
+  std::vector<RowAlt> alts; // ascending maxRows
   hfr_module *mod = nullptr;
   hipFunction_t fn = nullptr;
   hfr_launch_cfg cfg{};
@@ -191,8 +201,17 @@ int parseBlock(const std::vector<std::string> &lines, hfr_group &g) {
       if (!pl.cfg.grid[0] || !pl.cfg.block[0]) return fail(HFR_ERR_MANIFEST, "pre kernel without launch shape");
       g.pre.push_back(pl);
     }
+    else if (key == "alt") {
+      // alt <kernel> <max rows> <rows per block row> <blocks per block row> <threads>
+      RowAlt ra;
+      is >> ra.kernel >> ra.maxRows >> ra.rowsB >> ra.rowsC >> ra.block;
+      if (ra.maxRows <= 0 || ra.rowsB <= 0 || ra.rowsC <= 0 || !ra.block || (!g.alts.empty() && g.alts.back().maxRows >= ra.maxRows))
+        return fail(HFR_ERR_MANIFEST, "bad alt line: " + ln);
+      g.alts.push_back(ra);
+    }
     if (is.fail()) return fail(HFR_ERR_MANIFEST, "malformed manifest line: " + ln);
   }
+  if (!g.alts.empty() && !g.rowsDyn) return fail(HFR_ERR_MANIFEST, "alt kernels without rows_dyn");
   if (g.kernel.empty() || g.hsaco.empty()) return fail(HFR_ERR_MANIFEST, "manifest block without kernel/hsaco");
   if (!g.cfg.block[0] || !g.cfg.grid[0]) return fail(HFR_ERR_MANIFEST, "manifest block without launch shape");
   auto check = [&](const std::vector<Karg> &ks) {
@@ -280,12 +299,15 @@ int checkGroupArgs(const hfr_group *g, const uint64_t *params, size_t nparams, v
 // all on `stream`.
 int launchGroup(const hfr_group *g, const uint64_t *params, void *const *results, void *ws, void *stream,
                 int64_t rows = -1) {
-  auto launch = [&](hipFunction_t fn, hfr_launch_cfg cfg, const std::vector<Karg> &kargs) {
+  auto rowsCfg = [&](hfr_launch_cfg cfg) {
     if (g->rowsDyn && g->rowsA > 0) {
       int64_t blocks = (rows * g->rowsA + g->rowsB - 1) / g->rowsB * g->rowsC;
       if (g->rowsCap > 0 && blocks > g->rowsCap) blocks = g->rowsCap;
       cfg.grid[0] = (unsigned)(blocks > 0 ? blocks : 1);
     }
+    return cfg;
+  };
+  auto launch = [&](hipFunction_t fn, const hfr_launch_cfg &cfg, const std::vector<Karg> &kargs) {
     uint64_t args[HFR_MAX_KARGS];
     if (kargs.size() > HFR_MAX_KARGS) return fail(HFR_ERR_INVALID, "too many kernel arguments");
     size_t n = 0;
@@ -299,11 +321,19 @@ int launchGroup(const hfr_group *g, const uint64_t *params, void *const *results
     }
     return launchRaw(fn, cfg, args, n, stream);
   };
+  for (auto &alt : g->alts)
+    if (rows <= alt.maxRows) {
+      hfr_launch_cfg cfg{};
+      cfg.grid[0] = (unsigned)((rows + alt.rowsB - 1) / alt.rowsB * alt.rowsC);
+      cfg.grid[1] = cfg.grid[2] = cfg.block[1] = cfg.block[2] = 1;
+      cfg.block[0] = alt.block;
+      return launch(alt.fn, cfg, g->kargs);
+    }
   for (auto &pl : g->pre) {
     const int rc = launch(pl.fn, pl.cfg, pl.kargs);
     if (rc) return rc;
   }
-  return launch(g->fn, g->cfg, g->kargs);
+  return launch(g->fn, rowsCfg(g->cfg), g->kargs);
 }
 
 } // namespace
@@ -380,6 +410,8 @@ int hfr_group_load(const char *manifest_path, const char *func, hfr_group_t *out
   hipError_t e = hipModuleGetFunction(&g->fn, g->mod->mod, g->kernel.c_str());
   for (size_t i = 0; e == hipSuccess && i < g->pre.size(); ++i)
     e = hipModuleGetFunction(&g->pre[i].fn, g->mod->mod, g->pre[i].kernel.c_str());
+  for (size_t i = 0; e == hipSuccess && i < g->alts.size(); ++i)
+    e = hipModuleGetFunction(&g->alts[i].fn, g->mod->mod, g->alts[i].kernel.c_str());
   if (e != hipSuccess) {
     (void)hipGetLastError();
     hfr_module_unload(g->mod);

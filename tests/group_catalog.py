@@ -1258,6 +1258,13 @@ def entries():
     e["argmax_dyn_rt"] = g.with_dynamic_rows(g.argmax(333, 50000), 333)
     e["mx_fp4_dyn_rt"] = g.with_dynamic_rows(g.matmul_mx(333, 256, 512, fa="e2m1", fb="e2m1", via="bitcast",
                                                          name="mx_fp4_dyn"), 333)
+    # every contraction tile through one launch-time row count
+    for lay in ("nk", "kn"):
+        e[f"tiles_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 1088, b_layout=lay), 7919)
+        e[f"tiles_bf16_{lay}_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout=lay), 7919)
+    e["tiles_f16_kn_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout="kn", elem="f16"), 7919)
+    e["tiles_mx_e4m3_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 1040, 640, via="format"), 7919)
+    e["tiles_mx_e2m1_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 1040, 1280, fa="e2m1", fb="e2m1", via="format"), 7919)
     e["rmsnorm_quant_rank3"] = g.rmsnorm_quant(256, 1024, batch=4)
     # the same groups through the one-wave-per-row kernel (hf_rmsq.h, the
     # default for the widths it takes), named for it ...

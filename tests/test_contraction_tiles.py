@@ -1,0 +1,108 @@
+"""GPU: every tile of the contraction kernels.
+
+One code object per group takes the row count M at launch and runs the tile
+the lowering chooses for it (16x16 ... 256x128, then the 256x256 ring); N = 1040
+leaves every tile a ragged last column tile, K ends in half a 128-byte slice,
+and the row counts sit on and beside the tiles' edges.  Whole-number sums are
+exact; 16-bit floats are held to the f32 summation bound K 2^-24 sum|ab| plus
+half an ulp of the output; block-scaled results to the matrix core's bars.
+"""
+import numpy as np
+import pytest
+
+import hfusion_mi355x as hf
+import group_catalog as cat
+from test_dynamic import _call
+from test_matmul_mx import TOL_FP4, fp4_case, fp4_products
+
+I = hf.inputs
+N = 1040
+ROWS = [1, 16, 17, 33, 64, 65, 100, 129, 200, 2000, 3500, 5900]
+
+
+def test_alternatives_by_row_count():
+    """The manifest lists the kernels by ascending row count, each with the
+    grid of its tile, and they are what a static group of that M gets."""
+    for name, k, layout in (("tiles_w8a8_nk_rt", 1088, "nk"), ("tiles_w8a8_kn_rt", 1088, "kn")):
+        art = hf.compile(cat.get(name), options="dyn=runtime")
+        alts = [ln.split()[1:] for ln in open(art.manifest) if ln.startswith("alt ")]
+        rows = [int(a[1]) for a in alts]
+        assert rows == sorted(set(rows)) and len(alts) >= 5
+        for kern, top, rb, rc, threads in alts:
+            tm, tn = (int(v) for v in kern.rsplit("_", 1)[1].split("x"))
+            assert int(rb) == tm and int(rc) == (-(-N // tn) + 7) // 8 * 8 and int(threads) <= 1024
+            blk = hf.compile(hf.groups.w8a8_dequant(int(top), N, k, b_layout=layout), options="emit=hip").blocks[0]
+            assert f"{tm}x{tn} tiles" in blk["variant"]
+            assert blk["grid"][0] == -(-int(top) // tm) * int(rc)
+
+
+def _mm(rng, m, k, layout):
+    a = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    b = rng.integers(-127, 128, (N, k) if layout == "nk" else (k, N), dtype=np.int8)
+    bt = b.T if layout == "nk" else b
+    return a, b, (a.astype(np.float64) @ bt.astype(np.float64)).astype(np.int64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+def test_gpu_tiles_w8a8(gpu, layout):
+    rng = np.random.default_rng(77)
+    # (past 16384 rows the main kernel)
+    for m in ROWS + [16500] * (layout == "kn"):
+        print(f"[case] tiles_w8a8_{layout}_rt M={m}", flush=True)
+        a, b, c = _mm(rng, m, 1088, layout)
+        st, sc = rng.uniform(0.001, 0.02, m).astype(np.float32), rng.uniform(0.001, 0.02, N).astype(np.float32)
+        out, = _call(f"tiles_w8a8_{layout}_rt", [a, b, st, sc, np.zeros((m, N), np.uint16)], gpu)
+        ref = I.f32_to_bf16_bits((c.astype(np.float32) * st[:, None]) * sc[None, :])
+        assert np.array_equal(out.view(np.uint16), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elem,layout", [("bf16", "nk"), ("bf16", "kn"), ("f16", "kn")])
+def test_gpu_tiles_16bit(gpu, elem, layout):
+    rng, k = np.random.default_rng(78), 224
+    for m in ROWS:
+        print(f"[case] tiles_{elem}_{layout}_rt M={m}", flush=True)
+        fa, fb = rng.normal(0, 1, (m, k)).astype(np.float32), rng.normal(0, 1, (N, k) if layout == "nk" else (k, N)).astype(np.float32)
+        if elem == "bf16":
+            a, b = I.f32_to_bf16_bits(fa), I.f32_to_bf16_bits(fb)
+            fa, fb, up = I.bf16_bits_to_f32(a), I.bf16_bits_to_f32(b), 2.0 ** -8
+        else:
+            a, b = fa.astype(np.float16), fb.astype(np.float16)
+            fa, fb, up = a.astype(np.float32), b.astype(np.float32), 2.0 ** -11
+            a, b = a.view(np.uint16), b.view(np.uint16)
+        fa, fb = fa.astype(np.float64), (fb.T if layout == "nk" else fb).astype(np.float64)
+        out, = _call(f"tiles_{elem}_{layout}_rt", [a, b, np.zeros((m, N), np.uint16)], gpu)
+        got = (I.bf16_bits_to_f32(out.view(np.uint16)) if elem == "bf16" else out.view(np.float16)).astype(np.float64)
+        ref, bound = fa @ fb, k * 2.0 ** -24 * (np.abs(fa) @ np.abs(fb))
+        # the f32 sum is within `bound`, and rounding it moves it by up to half
+        # an ulp: 2^-8 of the value with bf16's 8 significant bits, 2^-11 with
+        # f16's 11
+        assert np.all(np.abs(got - ref) <= bound + up * (np.abs(ref) + bound) + 2.0 ** -25)
+
+
+@pytest.mark.gpu
+def test_gpu_tiles_mx_fp8(gpu):
+    rng, k = np.random.default_rng(79), 640
+    codes = np.array([c for c in range(256) if c & 0x7F != 0x7F], np.uint8)
+    import torch
+    dec = lambda u: torch.from_numpy(u).view(torch.float8_e4m3fn).float().numpy().astype(np.float64)
+    for m in ROWS[:-1]:
+        print(f"[case] tiles_mx_e4m3_rt M={m}", flush=True)
+        a, b = rng.choice(codes, (m, k)), rng.choice(codes, (k, N))
+        sa, sb = rng.integers(120, 131, (m, k // 32), dtype=np.uint8), rng.integers(120, 131, (N, k // 32), dtype=np.uint8)
+        out, = _call("tiles_mx_e4m3_rt", [a, b, sa, sb], gpu)
+        fa = dec(a) * np.repeat(np.exp2(sa.astype(np.float64) - 127), 32, axis=1)
+        fb = dec(b) * np.repeat(np.exp2(sb.astype(np.float64) - 127), 32, axis=1).T
+        assert np.all(np.abs(out - fa @ fb) <= 2.0 ** -11 * (np.abs(fa) @ np.abs(fb)))
+
+
+@pytest.mark.gpu
+def test_gpu_tiles_mx_fp4(gpu):
+    rng, k = np.random.default_rng(80), 1280
+    for m in ROWS[:-1]:
+        print(f"[case] tiles_mx_e2m1_rt M={m}", flush=True)
+        a, b, sa, sb, ca, cb = fp4_case(rng, m, N, k)
+        out, = _call("tiles_mx_e2m1_rt", [a, b, sa, sb], gpu)
+        mag, ref = fp4_products(ca, cb, sa, sb)
+        assert np.all(np.abs(out.astype(np.float64) - ref) <= TOL_FP4 * mag + 1e-30)
