@@ -3973,6 +3973,7 @@ struct RmsqMatch {
   size_t qRes = 0, sRes = 0;
   double s0 = 0, K = 0, eps = 0, a0 = 0, qd = 0;
   int lo = 0, hi = 0;
+  bool f32x = false; // x is f32, else bf16
 };
 
 const Op *defOp(const Value *v) { return v ? v->def : nullptr; }
@@ -4060,7 +4061,13 @@ bool matchRmsQuant(const Analysis &A, RmsqMatch &m) {
   const Op *y1 = defOp(ym->ins[0]);
   if (!binOp(y1, "mul")) return false;
   const Value *xf = y1->ins[0];
-  if ((m.x = bf16ArgCast(xf)) < 0) return false;
+  if ((m.x = bf16ArgCast(xf)) < 0) {
+    // an f32 x is a group argument itself
+    if (xf->argIdx < 0 || xf->type.elem != Elem::F32) return false;
+    m.x = xf->argIdx;
+    m.f32x = true;
+    if (A.map.at(xf) != std::vector<int>{0, 1}) return false;
+  }
   // inv = rec(sqrt(ss / K + eps)); ss = reduce addf (xf * xf) from s0
   const Value *inv = broadcastOf(y1->ins[1], {1});
   const Op *rc = defOp(inv);
@@ -4088,15 +4095,17 @@ KernelPlan lowerRmsQuant(Analysis &A, const RmsqMatch &m, const std::string &kna
   // one workgroup per CU: 12 waves, three per SIMD (the occupancy the
   // register budget allows); 12 row buffers and gamma fill 112 KB of LDS at
   // 4096 columns
-  constexpr int WPB = 12;
+  // (an f32 x: 8 waves, two per SIMD, 144 KB)
+  const int WPB = m.f32x ? 8 : 12;
+  const char *xt = m.f32x ? "float" : "uint16_t";
   KernelPlan p;
   p.kernelName = kname;
   p.kind = "LAST_AXIS_PBR";
   p.variant = "rmsnorm-quant: one wave per row, binade-run exact serial sum";
   std::ostringstream k;
-  k << "extern \"C\" __global__ __launch_bounds__(" << WPB * 64 << ") __attribute__((amdgpu_waves_per_eu(3))) void " << kname
+  k << "extern \"C\" __global__ __launch_bounds__(" << WPB * 64 << ") __attribute__((amdgpu_waves_per_eu(" << WPB / 4 << "))) void " << kname
     << "(" << kernelParamList(A, p.kargs, false) << ") {\n"
-    << "  hf::rmsq_rows<" << C << ", " << m.lo << ", " << m.hi << ", " << WPB << ">((const uint16_t*)p" << m.x
+    << "  hf::rmsq_rows<" << C << ", " << m.lo << ", " << m.hi << ", " << WPB << ", " << xt << ">((const " << xt << "*)p" << m.x
     << ", (const uint16_t*)p" << m.gamma << ", (int8_t*)" << resultPtr(A, m.qRes) << ", (float*)" << resultPtr(A, m.sRes)
     << ", " << (A.rowsDyn ? std::string("hf_rows") : std::to_string(R) + "ll") << ", " << floatLit((float)m.s0) << ", "
     << floatLit((float)m.K) << ", " << floatLit((float)m.eps) << ", "
@@ -4275,7 +4284,7 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
           rows = A.D.size() <= 2 && reducesLastDimOnly(A);
         }
         RmsqMatch rq;
-        if (rows && opt.rmsnKernel && matchRmsQuant(A, rq)) {
+        if (rows && opt.rmsnKernel && matchRmsQuant(A, rq) && !rq.f32x) {
           p = lowerRmsNorm(A, rq, kname);
         } else if (rows && opt.rmsqKernel && matchRmsQuant(A, rq)) {
           p = lowerRmsQuant(A, rq, kname);

@@ -9,8 +9,10 @@
 //   amax = maximumf over |y| from a0; scale = amax / QD;
 //   q = (int8) max(min(rint(y / scale), HI), LO).
 //
-// Exact serial sum.  Every addend x^2 of a bf16 x is exact in f32 and >= 0,
-// so the running sum never decreases.  While the running sum s stays inside
+// x is bf16 (xf above) or f32 (its own xf).
+//
+// Exact serial sum.  Every addend RN(x^2) is >= 0 (of a bf16 x it is exact in
+// f32), so the running sum never decreases.  While the running sum s stays inside
 // one binade [2^p, 2^(p+1)), each step is s' = s + (x^2 rounded to the binade's
 // grid u = 2^(p-23)), ties to even: in units of u, n' = n + d(n & 1).  A run of
 // steps inside one binade is therefore the map n -> n + D[n & 1], fixed by two
@@ -24,9 +26,9 @@
 //      binade p of every sub-segment; sub-segments whose prediction is not
 //      clear by a 2^-10 margin are marked dirty;
 //   3. for each clean sub-segment two candidate chains, started at 2^p (n = 0)
-//      and 2^p + u (n = 1), give D[0] and D[1]: fmaf(x, x, c) = RN(x^2 + c)
-//      because x^2 is exact (for |x| < 2^-63 the square is below half an ulp
-//      of c >= 2^-60 either way);
+//      and 2^p + u (n = 1), give D[0] and D[1]; of a bf16 x by fmaf(x, x, c) =
+//      RN(x^2 + c), because x^2 is exact (for |x| < 2^-63 the square is below
+//      half an ulp of c >= 2^-60 either way);
 //   4. runs (maximal sequences of clean sub-segments of one binade, in row
 //      order) compose inside the lane, then across lanes with a segmented
 //      scan over runs of whole lanes; a lane keeps an event per run that
@@ -40,6 +42,10 @@
 //      sub-segment.
 //   The result is the bit pattern of the serial sum for every input,
 //   including NaN and infinity (which always take the serial steps).
+// An f32 row is twice the bytes: 8 waves instead of 12 fill a CU's LDS.
+// Measured at 512 rows of 4096: 79.6 us -> 12.1 us for an f32 x, whose groups
+// ran the generic row program (32 rows per workgroup: 16 workgroups, each
+// row a chain of 4096 dependent adds).
 // Quantisation: y stays in registers; the row maximum is a wave reduction;
 // the int8 codes go through a bracketed fast path (exact recomputation of
 // near-tie words), a row whose Guard reports an unsafe magnitude is
@@ -138,12 +144,13 @@ __device__ __forceinline__ bool band_apply_packed(uint32_t &s, uint32_t w0, uint
 }
 
 // 16 serial steps s = RN(s + RN(x_k^2)) over lane j's elements x[0..15] (every
-// lane runs its own; lane j's result is returned).  From s >= 2^-100 on, one
-// FMA per step is the same: x^2 is exact unless |x| < 2^-63, and then it is
-// below half an ulp of s on both paths.
+// lane runs its own; lane j's result is returned).  Of a bf16 x (EXACT), from
+// s >= 2^-100 on, one FMA per step is the same: x^2 is exact unless |x| <
+// 2^-63, and then it is below half an ulp of s on both paths.
+template <bool EXACT>
 __device__ __forceinline__ uint32_t serial16(uint32_t s, const float *x, int j) {
   float sf = __uint_as_float(s);
-  if (s >= 0x0d800000u && s <= 0x7f800000u) { // [2^-100, inf]
+  if (EXACT && s >= 0x0d800000u && s <= 0x7f800000u) { // [2^-100, inf]
 #pragma unroll
     for (int k = 0; k < 16; ++k) sf = __builtin_fmaf(x[k], x[k], sf);
   } else {
@@ -188,15 +195,17 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-template <int C, int LO, int HI, int WPB>
-__device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const uint16_t *__restrict__ gamma,
+// XT: uint16_t (bf16 bits) or float, the element type of x
+template <int C, int LO, int HI, int WPB, typename XT>
+__device__ __forceinline__ void rmsq_rows(const XT *__restrict__ x, const uint16_t *__restrict__ gamma,
                                           int8_t *__restrict__ q, float *__restrict__ scale, int64_t R, float s0,
                                           float K, float eps, float a0, float qd, float *dbg = nullptr) {
   static_assert(C == 1024 || C == 2048 || C == 4096, "rows of 1024, 2048 or 4096 elements");
+  constexpr bool BF = sizeof(XT) == 2;
   constexpr int SEG = C / 64;      // elements per lane
-  constexpr int NG = SEG / 8;      // 16-byte granules per lane
+  constexpr int NG = SEG * (int)sizeof(XT) / 16; // 16-byte granules per lane
   constexpr int NS = SEG / 16;     // sub-segments per lane
-  __shared__ rq_u4 lds_all[WPB][C / 8];
+  __shared__ rq_u4 lds_all[WPB][C * sizeof(XT) / 16];
   const int lane0 = threadIdx.x & 63;
   rq_u4 *lds = lds_all[threadIdx.x / 64];
   // rows in rounds of W = grid * WPB: in a full round, wave w of workgroup b
@@ -223,28 +232,33 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
                                          __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
   }
   __syncthreads();
-  // row DMA straight into this wave's LDS row buffer.  Granule G (16 bytes,
-  // columns 8G .. 8G+7) of the row sits at slot G ^ ((G >> 4) & 7): a
-  // permutation inside every 128-byte line, so DMA instruction k, lane l
-  // fills slot 64k + l from one line per eight lanes (coalesced), and lane j's
-  // granule g (G = NG*j + g) is read with the 64 lanes spread over the banks.
-  // Slot 64k + l holds G = 64k + 8(l/8) + ((l % 8) ^ ((4k + l/16) & 7)); its
-  // byte offset is 1024k + off[k & 1] with off[1] = off[0] ^ 64.
+  // row DMA straight into this wave's LDS row buffer.  Granule G (16 bytes) of
+  // the row sits at slot G ^ ((G >> 4) & MASK): a permutation inside every
+  // 128-byte line (f32, whose lanes own more granules: inside every two), so
+  // DMA instruction k, lane l fills slot 64k + l from whole lines (coalesced),
+  // and lane j's granule g (G = NG*j + g) is read with 16 consecutive lanes on
+  // 16 (bf16: 8) different bank groups.  Slot 64k + l holds G = 64k + (l ^
+  // ((4k + l/16) & MASK)); its byte offset from row byte 1024k is off0 with
+  // bits 4 (k & (MASK >> 2)) of the granule flipped.
+  constexpr uint32_t MASK = BF ? 7 : NG - 1;
   const uint32_t ldsBase = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  const uint32_t dmaOff0 = 128u * (lane0 / 8) + 16u * ((lane0 % 8) ^ (lane0 / 16)), dmaOff1 = dmaOff0 ^ 64u;
+  const uint32_t dmaOff0 = 16u * ((uint32_t)lane0 ^ (((uint32_t)lane0 / 16) & MASK));
+  uint32_t dmaOff[MASK / 4 + 1];
+#pragma unroll
+  for (int k = 0; k < (int)(MASK / 4 + 1); ++k) dmaOff[k] = dmaOff0 ^ (64u * k);
   const rq_u4 *rdPtr[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const uint32_t G = NG * lane0 + g;
-    rdPtr[g] = lds + (G ^ ((G >> 4) & 7u));
+    rdPtr[g] = lds + (G ^ ((G >> 4) & MASK));
   }
   auto issueRow = [&](int64_t r) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's reads of the buffer are done
-    const uint16_t *rowp = x + uniform_i64(r) * C;
+    const char *rowp = reinterpret_cast<const char *>(x + uniform_i64(r) * C);
 #pragma unroll
     for (int k = 0; k < NG; ++k) {
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"((k & 1) ? dmaOff1 : dmaOff0),
-                   "s"(rowp + 512 * k), "s"(ldsBase + 1024u * k)
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(dmaOff[k & (MASK / 4)]),
+                   "s"(rowp + 1024 * k), "s"(ldsBase + 1024u * k)
                    : "memory");
     }
   };
@@ -275,8 +289,12 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
     for (int g = 0; g < NG; ++g)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        xf[8 * g + 2 * i] = __uint_as_float(seg[g][i] << 16);
-        xf[8 * g + 2 * i + 1] = __uint_as_float(seg[g][i] & 0xffff0000u);
+        if constexpr (BF) {
+          xf[8 * g + 2 * i] = __uint_as_float(seg[g][i] << 16);
+          xf[8 * g + 2 * i + 1] = __uint_as_float(seg[g][i] & 0xffff0000u);
+        } else {
+          xf[4 * g + i] = __uint_as_float(seg[g][i]);
+        }
       }
     float a[NS];
     float tot = 0.0f;
@@ -308,8 +326,14 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
       float c0 = __uint_as_float(base), c1 = __uint_as_float(base + 1u);
 #pragma unroll
       for (int k = 16 * t; k < 16 * t + 16; ++k) {
-        c0 = __builtin_fmaf(xf[k], xf[k], c0);
-        c1 = __builtin_fmaf(xf[k], xf[k], c1);
+        if constexpr (BF) {
+          c0 = __builtin_fmaf(xf[k], xf[k], c0);
+          c1 = __builtin_fmaf(xf[k], xf[k], c1);
+        } else {
+          const float sq = xf[k] * xf[k];
+          c0 = c0 + sq;
+          c1 = c1 + sq;
+        }
       }
       const uint32_t d0 = __float_as_uint(c0) - base, d1 = __float_as_uint(c1) - base - 1u;
       clean = clean && (d0 | d1) < (1u << 23);
@@ -324,7 +348,7 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
     // runs the steps over its own elements, lane 0's result is kept
     uint32_t p0 = __float_as_uint(s0);
 #pragma unroll
-    for (int t = 0; t < NS; ++t) p0 = serial16(p0, &xf[16 * t], 0);
+    for (int t = 0; t < NS; ++t) p0 = serial16<BF>(p0, &xf[16 * t], 0);
     // ---- 4. runs: maximal sequences of clean items of one binade, in row
     //         order.  Q[t] composes the run that ends at item t from its start
     //         in this lane; a segmented scan over the lanes composes the runs
@@ -394,7 +418,7 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
         if (a0 == 0x40000000u) {
           // a dirty item: its own serial steps (every lane runs its own
           // elements from s; lane j's result is kept)
-          s = serial16(s, &xf[16 * t], j);
+          s = serial16<BF>(s, &xf[16 * t], j);
           ++nslow;
           continue;
         }
@@ -416,7 +440,7 @@ __device__ __forceinline__ void rmsq_rows(const uint16_t *__restrict__ x, const 
 #pragma unroll
         for (int t = 0; t < NS; ++t) {
           if (!band_apply_packed(s, __builtin_amdgcn_readlane(w0[t], j), __builtin_amdgcn_readlane(w1[t], j))) {
-            s = serial16(s, &xf[16 * t], j);
+            s = serial16<BF>(s, &xf[16 * t], j);
             nslow += 1000;
           }
         }

@@ -1149,6 +1149,13 @@ def host_transpose_sum(m=300, n=64):
 """
 
 
+def rmsnorm_quant_f32(rows, cols):
+    """rmsnorm_quant with an f32 x (no widening cast)."""
+    lines = g.rmsnorm_quant(rows, cols).replace(f"%x: tensor<{rows}x{cols}xbf16>", f"%x: tensor<{rows}x{cols}xf32>").split("\n")
+    keep = [ln for ln in lines if not ln.lstrip().startswith(("%e0 =", "%xf ="))]
+    return "\n".join(keep).replace("%xf", "%x")
+
+
 def entries():
     """name -> IR text of every group the tests run: the product groups plus
     the parity cases below."""
@@ -1258,6 +1265,9 @@ def entries():
     e["argmax_dyn_rt"] = g.with_dynamic_rows(g.argmax(333, 50000), 333)
     e["mx_fp4_dyn_rt"] = g.with_dynamic_rows(g.matmul_mx(333, 256, 512, fa="e2m1", fb="e2m1", via="bitcast",
                                                          name="mx_fp4_dyn"), 333)
+    # the norm + quant pattern on an f32 x (as behind a contraction)
+    for c in (1024, 2048, 4096):
+        e[f"rmsnorm_quant_f32_{c}"] = rmsnorm_quant_f32(256, c)
     # every contraction tile through one launch-time row count
     for lay in ("nk", "kn"):
         e[f"tiles_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 1088, b_layout=lay), 7919)

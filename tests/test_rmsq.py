@@ -159,3 +159,37 @@ def test_rmsq_configs_bit_exact(gpu, name):
     rq, rs = run_oracle(name, args)
     assert np.array_equal(s.view(np.uint32), rs.view(np.uint32))
     assert np.array_equal(q, rq)
+
+
+def f32_rows(cols, seed):
+    """Rows of f32 values with full significands (their squares round): the
+    stress and fuzz kinds above, unrounded."""
+    rng = np.random.default_rng(0xF32 + seed)
+    base = I.bf16_bits_to_f32(np.concatenate([stress_rows(128, seed), fuzz_rows(128, seed)]))[:, :cols]
+    x = base * (1 + rng.uniform(-2.0 ** -9, 2.0 ** -9, base.shape) * (rng.random((256, 1)) < 0.8)).astype(np.float32)
+    return np.ascontiguousarray(x, np.float32)
+
+
+def test_rmsq_kernel_takes_f32():
+    for c in (1024, 2048, 4096):
+        ir = cat.get(f"rmsnorm_quant_f32_{c}")
+        assert "binade-run" in hf.compile(ir).blocks[0]["variant"]
+        assert "serial-order" in hf.compile(ir, options="rmsq_kernel=0").blocks[0]["variant"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [1024, 2048, 4096])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_rmsq_f32_bit_exact(gpu, cols, seed):
+    print(f"[case] rmsnorm_quant_f32_{cols} seed={seed}", flush=True)
+    name = f"rmsnorm_quant_f32_{cols}"
+    g = I.uniform_bf16(I.SEED_BASE + 79 + seed, (cols,), 0.25, 4.0)
+    args = [f32_rows(cols, seed), g, np.zeros((256, cols), np.int8), np.zeros(256, np.float32)]
+    q, s = run_gpu(name, args, gpu)
+    rq, rs = run_oracle(name, args)
+    nan = np.isnan(rs)
+    assert np.array_equal(np.isnan(s), nan)
+    assert np.array_equal(s[~nan].view(np.uint32), rs[~nan].view(np.uint32)), \
+        f"scales differ in rows {np.nonzero(s.view(np.uint32) != rs.view(np.uint32))[0][:16]}"
+    bad = np.nonzero((q != rq).any(axis=1))[0]
+    assert bad.size == 0, f"codes differ in rows {bad[:16]}"
