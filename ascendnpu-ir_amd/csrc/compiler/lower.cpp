@@ -2276,7 +2276,12 @@ KernelPlan lowerReduceWithIndex(Analysis &A, const std::string &kname) {
     segs = rows >= CUS ? 1 : std::max<int64_t>(1, (2 * CUS + rows - 1) / rows);
     segLen = ((C + segs - 1) / segs + 3) / 4 * 4;
     segLen = std::max<int64_t>(segLen, std::min<int64_t>((C + 3) / 4 * 4, 4096)); // no tiny segments
+    if (segs > 1) segLen = std::min<int64_t>(segLen, int64_t(1) << 29); // a record's position has 30 bits
     segs = (C + segLen - 1) / segLen;
+    if (segs > 512) { // (the fold holds 512 records)
+      segs = 1;
+      segLen = (C + 3) / 4 * 4;
+    }
   };
   int64_t segs, segLen;
   schedule(A.rowsDyn ? CUS : R, segs, segLen);
@@ -2295,7 +2300,7 @@ KernelPlan lowerReduceWithIndex(Analysis &A, const std::string &kname) {
     for (int64_t r = 1; r < CUS; ++r) {
       int64_t sg, sl;
       schedule(r, sg, sl);
-      ws = std::max<uint64_t>(ws, (uint64_t)(r * sg * 16 + r * 4 + 256));
+      ws = std::max<uint64_t>(ws, (uint64_t)(r * sg * 8 + r * 128 + 256));
     }
     p.variant = "runtime rows: split rows below one per CU, a workgroup per row above";
     k << "extern \"C\" __global__ __launch_bounds__(" << BLOCK << ") void " << kname << "("
@@ -2331,7 +2336,7 @@ KernelPlan lowerReduceWithIndex(Analysis &A, const std::string &kname) {
   p.grid[0] = (unsigned)(R * segs);
   p.block[0] = BLOCK;
   // workspace: per-segment partial records + one arrival counter per row
-  p.workspaceBytes = (uint64_t)(R * segs * 16 + R * 4 + 256);
+  p.workspaceBytes = (uint64_t)(R * segs * 8 + R * 128 + 256);
   p.workspaceZeroInit = true;
   return p;
 }

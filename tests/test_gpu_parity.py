@@ -110,6 +110,41 @@ def test_argmax(gpu, name, rows, cols, it):
     assert np.array_equal(v[ok].view(np.uint32), rv[ok].view(np.uint32))
 
 
+@pytest.mark.parametrize("name,rows,cols", [("argmax_16", 16, 152064), ("argmax_row", 1, 2100004)])
+def test_argmax_split_rows(gpu, name, rows, cols):
+    """What the fold of a row's segment records has to get right, each case
+    twice in a row through one workspace: NaNs before and after the maximum in
+    its segment and in others, several of them, zeros of both signs and equal
+    maxima in different segments, rows without a value above the init."""
+    rng = np.random.default_rng(31)
+    at = [int(f * cols) for f in (0.0, 0.03, 0.31, 0.5, 0.97)] + [cols - 1]
+    art = hf.compile(cat.get(name), options=cat.options(name), require_cached=True)
+    import torch
+    grp = art.load()
+    for case in range(8 if rows == 1 else 1):
+        note(f"{name} split case {case}")
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        for r in range(rows):
+            k = (r + case) % 8
+            if k == 1: x[r, at[2]] = np.nan
+            if k == 2: x[r, at[4]], x[r, at[3]], x[r, at[3] + 5] = np.nan, np.nan, 9.0
+            if k == 3: x[r, at[3]], x[r, at[3] + 5] = 9.0, np.nan
+            if k == 4: x[r], x[r, at[1]], x[r, at[4]] = -1.0, -0.0, 0.0
+            if k == 5: x[r, at[1]] = x[r, at[2]] = x[r, at[5]] = 9.0
+            if k == 6: x[r] = -np.inf
+            if k == 7: x[r, 0] = np.nan
+        rv, ri = run_oracle(name, [x, zeros(rows, np.float32), zeros(rows, np.int32)])
+        xd = torch.from_numpy(x).to(gpu)
+        for _ in range(2):
+            v, i = torch.full((rows,), 7.0, device=gpu), torch.full((rows,), 7, dtype=torch.int32, device=gpu)
+            grp(xd, v, i)
+            torch.cuda.synchronize()
+            v, i = v.cpu().numpy(), i.cpu().numpy()
+            assert np.array_equal(i, ri) and np.array_equal(np.isnan(v), np.isnan(rv))
+            ok = ~np.isnan(rv)
+            assert np.array_equal(v[ok].view(np.uint32), rv[ok].view(np.uint32))
+
+
 def test_argmax_repeat_launch(gpu):
     """The per-row arrival counters reset themselves: two launches agree."""
     note("argmax_16 repeated")
