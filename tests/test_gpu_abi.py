@@ -242,3 +242,43 @@ def test_group_launcher_repeats_the_launch(gpu):
         ref, = run_oracle("safe_softmax_ragged", [xs, np.zeros((rows, cols), np.uint16)])
         d = bf16_ulp_diff(to_host(o, p[1]["elem"]), ref)
         assert d.max() <= 1, (k, int(d.max()))
+
+
+def test_plain_call_checks_and_stream(gpu):
+    """A call with no options: what it refuses (with the same errors as a call
+    with options), a launch-time row count that changes between calls, an
+    untied result, and the current stream."""
+    import torch
+    grp = hf.compile(cat.get("vec_add_1m"), require_cached=True).load()
+    a, b, o = (torch.ones(1 << 20, device=gpu) for _ in range(3))
+    assert grp(a, b, o) is o and float(o[-1]) == 2.0
+    for bad, err in (((a, b), TypeError), ((a, b.half(), o), ValueError), ((a, b[:-1], o), ValueError),
+                     ((a, b.cpu(), o), TypeError), ((a, 3, o), TypeError),
+                     ((a, torch.ones(1 << 21, device=gpu)[::2], o), ValueError)):
+        for kw in ({}, {"stream": 0}):
+            with pytest.raises(err):
+                grp(*bad, **kw)
+    dg = hf.DynamicGroup(cat.get("w8a8_dyn_rt"), require_cached=True, runtime=True)
+    wt = torch.randint(-9, 9, (512, 512), dtype=torch.int8, device=gpu)
+    for rows in (3, 40, 3):
+        x = torch.randint(-9, 9, (rows, 512), dtype=torch.int8, device=gpu)
+        st, sc = torch.ones(rows, device=gpu), torch.ones(512, device=gpu)
+        out = dg(x, wt, st, sc, torch.empty(rows, 512, dtype=torch.bfloat16, device=gpu))
+        assert torch.equal(out, (x.double() @ wt.double().t()).bfloat16())
+        with pytest.raises(ValueError):
+            dg(x, wt, torch.ones(rows + 1, device=gpu), sc, out)
+    mx = hf.compile(cat.get("mx_e4m3"), require_cached=True).load()
+    p = mx.meta["params"]
+    args = [torch.zeros(q["shape"], dtype=hf.torch_dtype(q["elem"]), device=gpu) for q in p]
+    r1, r2 = mx(*args), mx(*args)
+    assert r1.data_ptr() != r2.data_ptr() and r1.shape == (256, 256)
+    side = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20000000)
+        o.fill_(0)
+        grp(a, b, o)  # after the fill, on the side stream
+        done = torch.cuda.Event()
+        done.record()
+    assert not done.query()
+    side.synchronize()
+    assert float(o.min()) == 2.0
