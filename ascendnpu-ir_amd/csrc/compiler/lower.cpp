@@ -1235,6 +1235,7 @@ struct RowEmitter {
   bool afterOrdered = false;
   std::map<std::string, size_t> declaredAt; // array -> body offset of its declaration (pre: 0)
   int64_t R = 1, C = 1;
+  int64_t rowsHint = 0; // rows the serial-order schedule is made for (R unless set)
   int TR = 64, RB = 1, RPW = 1, VEC = 4, EPL = 4, CH = 0;
   bool masked = false;
 
@@ -1347,6 +1348,7 @@ struct RowEmitter {
     if (A.D.size() == 2) { R = A.D[0]; C = A.D[1]; }
     else if (A.D.size() == 1) { R = 1; C = A.D[0]; }
     else throw CompileError("row programs support rank-1 and rank-2 groups");
+    if (!rowsHint) rowsHint = R;
     // vector width from the tensors that travel through HBM
     int maxBytes = 1;
     auto consider = [&](const Value *v) {
@@ -1358,16 +1360,24 @@ struct RowEmitter {
     for (auto *r : A.f->returns) consider(r);
     VEC = std::max(1, 16 / maxBytes);
     if (VEC > 8) VEC = 8;
-    while (VEC > 1 && C % VEC) VEC /= 2;
+    // (a row length that is no multiple of VEC keeps the width: rows then
+    // start on any element and the last chunk is masked.  Softmax, 4096 rows
+    // of 32767: 181 -> 147 us, of 5003 33.9 -> 25.9)
     if (needOrdered) {
-      // one wave per row group, 4 rows each, 8 waves: 32 rows per block with
-      // a single serial chain lane per row in wave 0 (2 waves per SIMD leave
-      // 256 VGPRs per lane for the resident rows)
+      // one wave per row group of up to 4 rows, up to 8 waves: at most 32 rows
+      // per block with a single serial chain lane per row in wave 0 (2 waves
+      // per SIMD leave 256 VGPRs per lane for the resident rows).  A row's
+      // chain takes as long alone as beside others, so a block has no more
+      // rows than give every CU a block: 32 rows a block against this rule,
+      // softmax rows x 4096: 16 42 -> 17.6 us, 1000 48.8 -> 19.2, 2048 49.9 ->
+      // 22.6, 4096 56 -> 33; norm + quant 256 x 3072 23.5 -> 13.5
       TR = 64;
-      RB = 8;
-      RPW = 4;
+      RB = rowsHint <= 256 ? 1 : rowsHint <= 512 ? 2 : rowsHint <= 1024 ? 4 : 8;
+      RPW = rowsHint <= 2048 ? 1 : rowsHint <= 4096 ? 2 : 4;
     } else {
-      int64_t perLaneTarget = VEC * 4;
+      // 128 bytes of a lane's row in flight (softmax, 4096 rows of 9544: 49.6
+      // -> 42.3 us against 64 bytes; 777 rows of 5003 8.5 -> 7.6)
+      const int64_t perLaneTarget = VEC * 8 < 32 ? VEC * 8 : 32;
       int tr = 64;
       while (tr < 1024 && (int64_t)tr * perLaneTarget < C) tr *= 2;
       TR = tr;
@@ -4296,6 +4306,15 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
         } else if (rows) {
           RowEmitter e(A, opt);
           p = e.run(kname, "LAST_AXIS_PBR");
+          // a launch-time row count: the serial-order schedules for fewer rows
+          if (A.rowsDyn && e.needOrdered)
+            for (int64_t rows : {256, 512, 1024, 2048, 4096}) {
+              RowEmitter few(A, opt);
+              few.rowsHint = rows;
+              const KernelPlan q = few.run(kname + "_r" + std::to_string(rows), "LAST_AXIS_PBR");
+              p.source += q.source;
+              p.alts.push_back({q.kernelName, rows, q.rowsB, 1, q.block[0]});
+            }
         } else {
           collapseDomain(A);
           ColumnEmitter e(A);

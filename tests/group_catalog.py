@@ -1261,6 +1261,8 @@ def entries():
     # one kernel for every row count (compiler option dyn=runtime)
     e["rmsnorm_quant_dyn_rt"] = e["rmsnorm_quant_dyn"]
     e["softmax_dyn_rt"] = e["softmax_dyn"]
+    for c in (603, 1000):  # serial-order row schedules by row count, odd and whole chunks
+        e[f"rmsnorm_quant_w{c}_rt"] = g.with_dynamic_rows(g.rmsnorm_quant(7919, c), 7919)
     e["eltwise_mix_dyn_rt"] = g.with_dynamic_rows(eltwise_mix(67, 1000), 67)
     e["w8a8_dyn_rt"] = g.with_dynamic_rows(g.w8a8_dequant(333, 512, 512), 333)
     e["argmax_dyn_rt"] = g.with_dynamic_rows(g.argmax(333, 50000), 333)

@@ -359,3 +359,20 @@ def test_gpu_runtime_rows_argmax(gpu, rows):
     assert np.array_equal(v.view(np.uint32), rv.view(np.uint32)) or \
         (np.array_equal(np.isnan(v), np.isnan(rv)) and np.array_equal(v[~np.isnan(v)], rv[~np.isnan(rv)]))
     assert np.array_equal(i, ri)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [603, 1000])
+def test_gpu_row_schedules(gpu, cols):
+    """The serial-order row program's schedules (1 to 32 rows a block), the one
+    for each row count through one code object, at the counts where they
+    change and one row past: bit-exact codes and scales."""
+    rng = np.random.default_rng(90 + cols)
+    for rows in (1, 256, 257, 513, 1025, 2049, 4097):
+        note(f"rmsnorm_quant_w{cols}_rt rows={rows}")
+        x = (rng.standard_normal((rows, cols)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        g = (rng.uniform(0.5, 1.5, cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        args = [x, g, np.zeros((rows, cols), np.int8), np.zeros(rows, np.float32)]
+        q, s = _call(f"rmsnorm_quant_w{cols}_rt", args, gpu)
+        rq, rs = run_oracle(f"rmsnorm_quant_w{cols}_rt", args)
+        assert np.array_equal(q, rq) and np.array_equal(s.view(np.uint32), rs.view(np.uint32))
