@@ -206,7 +206,7 @@ __device__ __forceinline__ void mm_epilogue(acc_t (&acc)[4][4], typename Epi::ou
 // 32*JT columns.  When the whole 256x256 tile fits the stage (2-byte
 // outputs) all waves compute at once; otherwise the two row halves (waves
 // wm = 0, then wm = 1) take turns.
-template <typename Epi, int JT = 4, int NT = 256, typename acc_t, typename Args>
+template <typename Epi, int JT = 4, int NT = 256, bool AGPR = true, typename acc_t, typename Args>
 __device__ __forceinline__ void mm_epilogue_lds(acc_t (&acc)[4][JT], typename Epi::out_t *__restrict__ out, int64_t M,
                                                 int64_t N, int64_t m0, int64_t n0, int wm, int wn, int lane, const Args &P,
                                                 char *stage, int stage_bytes) {
@@ -242,7 +242,9 @@ __device__ __forceinline__ void mm_epilogue_lds(acc_t (&acc)[4][JT], typename Ep
             const int64_t n = n0 + col;
             const typename Epi::col_t cv = Epi::col(FULL || n < N ? n : N - 1, P);
             acc_t a = acc[i][j];
-            asm volatile("" : "+a"(a)::"memory"); // one tile in VGPRs at a time
+            // one tile's values computed at a time
+            if constexpr (AGPR) asm volatile("" : "+a"(a)::"memory");
+            else asm volatile("" : "+v"(a)::"memory");
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
               const int row = i * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
@@ -539,34 +541,18 @@ constexpr int MMD2_SLICE = 256 * 128;
 // k-row k0 + j/2 at column c0 + 8 (j % 2) gives lane i the column c0 + i at
 // k-rows k0 .. k0+7 -- eight consecutive k-bytes of one column, as the matrix
 // core takes them.
-// Block-scaled fp8 (MK_MX..): B [K, N] as above; SA [M, K/32] and SB
-// [N, K/32] hold the e8m0 scales.  One 128-byte slice is 2 scaled MFMAs of
-// 64 k per tile, each taking the int8 path's fragments of two k-blocks.  The
-// slice's scales (bytes 4s .. 4s+3 of each row: 1 KB for the tile's 256 A
-// rows, 1 KB for its 256 B columns) ride the same ring, one 4-byte-per-lane
-// DMA per wave per stage, so every load of a stage is covered by the ring's
-// own wait.  Block-scaled fp4 (MK_MX4): a 128-byte slice holds 256 k, four
-// scaled fp4 MFMAs of 64 k per tile, each taking the int8 path's fragment of
-// one k-block (16 bytes, 32 k per lane); the slice's scales are 8 bytes of
-// each row, two 4-byte DMAs per wave per stage into two planes.
 // AKM: A is [K, M] (hivm a_transpose), staged and read exactly as a [K, N] B
 // (its M columns in place of N).
 template <int MK, typename Epi, bool BKN, bool AKM = false, typename ElemT, typename Args>
 __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restrict__ B, typename Epi::out_t *__restrict__ out,
-                             int64_t M, int64_t N, int64_t K, const Args &P, const uint8_t *__restrict__ SA = nullptr,
-                             const uint8_t *__restrict__ SB = nullptr) {
-  constexpr bool MX = mk_is_mx(MK), FP4 = mk_is_fp4(MK);
-  constexpr int NW = FP4 ? 2 : 1; // scale words per row per stage (32 k per byte)
-  static_assert(!AKM || !MX, "block-scaled A is [M, K]");
-  static_assert(!(BKN || AKM) || (((MK == MK_I8 || MX) && sizeof(ElemT) == 1) ||
+                             int64_t M, int64_t N, int64_t K, const Args &P) {
+  static_assert(!(BKN || AKM) || ((MK == MK_I8 && sizeof(ElemT) == 1) ||
                                   ((MK == MK_BF16 || MK == MK_F16) && sizeof(ElemT) == 2)),
                 "the K-major operand path takes bytes or 16-bit floats");
-  static_assert(!MX || BKN, "block-scaled operands come with B [K, N]");
-  using Op = typename std::conditional<MX, MfmaMx<(MX ? MK : MK_MX)>, MfmaOp<(MX ? MK_I8 : MK)>>::type;
+  using Op = MfmaOp<MK>;
   using acc_t = typename Op::acc_t;
   constexpr int ESZ = sizeof(ElemT);
   __shared__ __attribute__((aligned(1024))) char lds[2][2][MMD2_SLICE]; // [stage][A/B]
-  __shared__ __attribute__((aligned(1024))) uint32_t lds_sc[MX ? 2 : 1][2 * NW][MX ? 256 : 1]; // [stage][A/B x word][row]
   const int tmt = (int)((M + MM_TM - 1) / MM_TM), tnt = (int)((N + MM_TN - 1) / MM_TN);
   int ti, tj;
   mm_tile_of(blockIdx.x, tmt, tnt, ti, tj);
@@ -574,7 +560,7 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
   const int64_t Kb = K * ESZ;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int wm = wave / 4, wn = wave % 4; // waves w and w+4 share a SIMD
-  constexpr int DPS = 8 + (MX ? NW : 0); // DMA instructions per wave per stage
+  constexpr int DPS = 8; // DMA instructions per wave per stage
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&lds[0][0][0];
   const char *Ab = reinterpret_cast<const char *>(A), *Bb = reinterpret_cast<const char *>(B);
   const int nsteps = (int)(Kb / 128);
@@ -636,26 +622,9 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
                         (uint32_t)((wave * 4 + (d & 3)) * 1024);
     mmd_dma16_off(dbase[d >= 4] + (int64_t)s * dstride[d >= 4], dofs[d], __builtin_amdgcn_readfirstlane(st));
   };
-  // the scales of K slice s: wave w carries 64 rows (w < 4: A rows 64 w ..,
-  // else B columns 64 (w - 4) ..), 4 bytes each (fp4: 8 bytes, as two words
-  // in two planes); a row of scales has K/32 bytes (fp4: K/16, K in bytes)
-  const uint32_t lds_sc0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)&lds_sc[0][0][0];
-  auto issue_scales = [&](int s, int slot) {
-    if constexpr (MX) {
-      const int op = wave / 4, r = 64 * (wave % 4) + lane;
-      const int64_t rows = op ? N : M, row0 = op ? n0 : m0;
-      int64_t row = row0 + r;
-      row = row < rows ? row : rows - 1;
-#pragma unroll
-      for (int w = 0; w < NW; ++w)
-        mmd_dma4((op ? SB : SA) + row * (K / (32 / NW)) + 4 * NW * (int64_t)s + 4 * w,
-                 __builtin_amdgcn_readfirstlane(lds_sc0 + (uint32_t)(((slot * 2 + op) * NW + w) * 1024 + 256 * (wave % 4))));
-    }
-  };
   auto issue_stage = [&](int s) {
 #pragma unroll
     for (int d = 0; d < 8; ++d) issue_one(s < nsteps ? s : nsteps - 1, s & 1, d);
-    issue_scales(s < nsteps ? s : nsteps - 1, s & 1);
   };
 
   acc_t acc[4][2];
@@ -724,20 +693,6 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
     }
   };
 
-  // this lane's scale words for stage s, shifted so that byte 2h is the scale
-  // of its k-half in half h of the slice (fp4: word w, byte 2q, of its
-  // k-half in k-block 2w + q; word 1 is read for the second half, after the
-  // first half's fragments are dead)
-  uint32_t sa_w[4], sb_w[2];
-  auto read_scales = [&](int s, int w) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      sa_w[i] = lds_sc[MX ? (s & 1) : 0][w][MX ? wm * 128 + i * 32 + lane % 32 : 0] >> (8 * (lane / 32));
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      sb_w[j] = lds_sc[MX ? (s & 1) : 0][NW + w][MX ? (wn * 2 + j) * 32 + lane % 32 : 0] >> (8 * (lane / 32));
-  };
-
   // Step s: wait for stage s (stage s+1 may be in flight); multiply its first
   // half while reading the second half's fragments; after a barrier (all of
   // stage s is in registers everywhere) issue stage s+2 into the freed slot
@@ -752,76 +707,274 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
     __syncthreads();
     fetch(s, 0, f0);
     fetch(s, 1, f1);
-    if constexpr (FP4) {
-      // k-blocks 0 and 1 of the slice: one scaled fp4 MFMA each
-      read_scales(s, 0);
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = q == 0 ? Op::template run<0>(mx_lo(f0[0][i]), mx_lo(f0[0][4 + j]), acc[i][j], (int)sa_w[i], (int)sb_w[j])
-                               : Op::template run<2>(mx_lo(f0[1][i]), mx_lo(f0[1][4 + j]), acc[i][j], (int)sa_w[i], (int)sb_w[j]);
-    } else if constexpr (MX) {
-      read_scales(s, 0);
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = Op::template run<0>(mx_cat(f0[0][i], f0[1][i]), mx_cat(f0[0][4 + j], f0[1][4 + j]), acc[i][j],
-                                          (int)sa_w[i], (int)sb_w[j]);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = Op::run(f0[q][i], f0[q][4 + j], acc[i][j]);
-    }
+        for (int j = 0; j < 2; ++j) acc[i][j] = Op::run(f0[q][i], f0[q][4 + j], acc[i][j]);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads(); // every wave holds stage s in registers: its slot is free
     const int s2 = s + 2 < nsteps ? s + 2 : nsteps - 1;
-    if constexpr (FP4) {
-      // k-blocks 2 and 3
-      read_scales(s, 1);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          __builtin_amdgcn_sched_barrier(0);
-          issue_one(s2, s & 1, i * 2 + j);
-          acc[i][j] = Op::template run<0>(mx_lo(f1[0][i]), mx_lo(f1[0][4 + j]), acc[i][j], (int)sa_w[i], (int)sb_w[j]);
-          acc[i][j] = Op::template run<2>(mx_lo(f1[1][i]), mx_lo(f1[1][4 + j]), acc[i][j], (int)sa_w[i], (int)sb_w[j]);
-        }
-      issue_scales(s2, s & 1);
-    } else if constexpr (MX) {
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        issue_one(s2, s & 1, q * 4 + i);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          __builtin_amdgcn_sched_barrier(0);
-          issue_one(s2, s & 1, i * 2 + j);
-          acc[i][j] = Op::template run<2>(mx_cat(f1[0][i], f1[1][i]), mx_cat(f1[0][4 + j], f1[1][4 + j]), acc[i][j],
-                                          (int)sa_w[i], (int)sb_w[j]);
-        }
-      issue_scales(s2, s & 1);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          __builtin_amdgcn_sched_barrier(0);
-          issue_one(s2, s & 1, q * 4 + i);
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = Op::run(f1[q][i], f1[q][4 + j], acc[i][j]);
-        }
-    }
+        for (int j = 0; j < 2; ++j) acc[i][j] = Op::run(f1[q][i], f1[q][4 + j], acc[i][j]);
+      }
     __builtin_amdgcn_sched_barrier(0);
   }
   mmd_wait_vm<0>();
   __syncthreads();
   mm_epilogue_lds<Epi, 2, 512>(acc, out, M, N, m0, n0, wm, wn, lane, P, &lds[0][0][0], (int)sizeof(lds));
+}
+
+// ---- DMA path, 128-byte K slices, alternating wave groups ---------------------
+// The 256x256 tile of mmad_core_pp with its two waves per SIMD taking turns:
+// waves 0-3 (group 0, rows 0-127) multiply while waves 4-7 (group 1, rows
+// 128-255) read fragments and issue DMAs, then the other way round, one
+// barrier between turns.  A slice is two turns of 16 multiplies (512 cycles)
+// per group, by row halves: M0 reads all of B's and the first 64 A rows'
+// fragments, C0 multiplies them, M1 reads the other 64 rows', C1 multiplies.
+//   phase   4s-1   4s    4s+1   4s+2   4s+3
+//   group 0 M0(s)  C0(s) M1(s)  C1(s)  M0(s+1)
+//   group 1        M0(s) C0(s)  M1(s)  C1(s)
+// B and the first row halves of slice s have been read by the end of phase
+// 4s: their part of slice s+2 (batch 1, 6 DMAs per wave) is issued in M1(s);
+// the second row halves by the end of phase 4s+2: batch 2 (2 per wave) of slice
+// s+2 is issued in M0(s+1).  Each has five to six phases until it is read.  At the
+// end of every even phase a wave waits until at most its last 8 DMAs are in
+// flight: then what the next phases read has landed (slices past the end
+// re-read the last one into regions no longer read, so the count holds).
+// Block-scaled fp8 (MK_MX..): B [K, N] as above; SA [M, K/32] and SB
+// [N, K/32] hold the e8m0 scales.  One 128-byte slice is 2 scaled MFMAs of
+// 64 k per tile, each taking the int8 path's fragments of two k-blocks.  The
+// slice's scales (bytes 4s .. 4s+3 of each row: 1 KB for the tile's 256 A
+// rows, 1 KB for its 256 B columns) ride the same ring, one 4-byte-per-lane
+// DMA per wave per stage, so every load of a stage is covered by the ring's
+// own wait.  Block-scaled fp4 (MK_MX4): a 128-byte slice holds 256 k, four
+// scaled fp4 MFMAs of 64 k per tile, each taking the int8 path's fragment of
+// one k-block (16 bytes, 32 k per lane); the slice's scales are 8 bytes of
+// each row, two 4-byte DMAs per wave per stage into two planes.
+// No value is pinned to an accumulation register: without one in the kernel
+// the compiler keeps all 256 registers of a wave as one file, where the pinned
+// form split them 128 / 128 and copied a block-scaled accumulator tile in and
+// out every step (and spilled 64 registers of this kernel).
+// Measured at 4096^3 against mmad_core_pp, one box: W8A8 64.7 -> 62.3 us, bf16
+// 107.8 -> 102.6, block-scaled fp8 75.0 -> 72.5, fp4 54.5 -> 53.4.  What bounds it
+// is power: with all operands zero the same launches take 38.7 (pp: 44.5), 66.0
+// (77.8) and 58.5 us (63.3); multiplies and barriers alone, without DMAs and
+// fragment reads, take 53 us on random int8.
+template <int MK, typename Epi, bool BKN, typename ElemT, typename Args>
+__device__ void mmad_core_alt(const ElemT *__restrict__ A, const ElemT *__restrict__ B, typename Epi::out_t *__restrict__ out,
+                              int64_t M, int64_t N, int64_t K, const Args &P, const uint8_t *__restrict__ SA = nullptr,
+                              const uint8_t *__restrict__ SB = nullptr) {
+  constexpr bool MX = mk_is_mx(MK), FP4 = mk_is_fp4(MK);
+  constexpr int NW = MX ? (FP4 ? 2 : 1) : 0; // scale words per row per stage
+  static_assert(!MX || BKN, "block-scaled operands come with B [K, N]");
+  using Op = typename std::conditional<MX, MfmaMx<(MX ? MK : MK_MX)>, MfmaOp<(MX ? MK_I8 : MK)>>::type;
+  using acc_t = typename Op::acc_t;
+  constexpr int ESZ = sizeof(ElemT);
+  __shared__ __attribute__((aligned(1024))) char lds[2][2][MMD2_SLICE]; // [stage][A/B]
+  __shared__ __attribute__((aligned(1024))) uint32_t lds_sc[MX ? 2 : 1][2 * (MX ? NW : 1)][MX ? 256 : 1]; // [stage][A/B x word][row]
+  const int tmt = (int)((M + MM_TM - 1) / MM_TM), tnt = (int)((N + MM_TN - 1) / MM_TN);
+  int ti, tj;
+  mm_tile_of(blockIdx.x, tmt, tnt, ti, tj);
+  const int64_t m0 = (int64_t)ti * MM_TM, n0 = (int64_t)tj * MM_TN;
+  const int64_t Kb = K * ESZ;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int wm = wave / 4, wn = wave % 4; // waves w and w+4 share a SIMD; wm is the group
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&lds[0][0][0];
+  const char *Ab = reinterpret_cast<const char *>(A), *Bb = reinterpret_cast<const char *>(B);
+  const int nsteps = (int)(Kb / 128);
+  auto kn_swz = [](int kr) { return ESZ == 1 ? ((kr & 7) << 1) | ((kr >> 3) & 1) : (kr & 3) << 2; };
+
+  // DMA d of a stage: 0-3 B, 4-5 the first row halves of A (rows 0-63 and
+  // 128-191), 6-7 the second; sources and layouts as in mmad_core_pp
+  uint32_t dofs[8];
+  int dblk[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    const int h = wave * 2 + (d & 1);
+    const int blk = d < 4 ? wave * 4 + d : h / 8 * 16 + h % 8 + (d >= 6 ? 8 : 0);
+    dblk[d] = blk;
+    if (d < 4 && BKN) {
+      const int LR = ESZ == 1 ? 16 : 32; // lanes per k-row
+      const int kr = (64 / LR) * blk + lane / LR, gg = (lane % LR) ^ kn_swz(kr);
+      int64_t col = n0 + gg * (16 / ESZ);
+      col = col + 16 / ESZ <= N ? col : N - 16 / ESZ;
+      dofs[d] = (uint32_t)((kr * N + col) * ESZ);
+    } else {
+      const int r = 8 * blk + lane / 8, g = (lane % 8) ^ ((r >> 1) & 7);
+      const int64_t rows = d < 4 ? N : M, row0 = d < 4 ? n0 : m0;
+      int64_t row = row0 + r;
+      row = row < rows ? row : rows - 1;
+      dofs[d] = (uint32_t)((row - row0) * Kb + g * 16);
+    }
+  }
+  const char *const abase = Ab + m0 * Kb, *const bbase = BKN ? Bb : Bb + n0 * Kb;
+  const int64_t bstride = BKN ? 128 * N : 128;
+  const uint32_t lds_sc0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)&lds_sc[0][0][0];
+  auto issue = [&](int s, int d) { // slice s (clamped) into slot s & 1
+    const int sk = s < nsteps ? s : nsteps - 1;
+    const uint32_t st = lds0 + (uint32_t)((s & 1) * 2 * MMD2_SLICE) + (d < 4 ? (uint32_t)MMD2_SLICE : 0u) + (uint32_t)(dblk[d] * 1024);
+    mmd_dma16_off(d < 4 ? bbase + (int64_t)sk * bstride : abase + (int64_t)sk * 128, dofs[d], __builtin_amdgcn_readfirstlane(st));
+  };
+  auto issue_scales = [&](int s) {
+    if constexpr (MX) {
+      const int sk = s < nsteps ? s : nsteps - 1, op = wave / 4;
+      const int64_t rows = op ? N : M, row0 = op ? n0 : m0;
+      int64_t row = row0 + 64 * (wave % 4) + lane;
+      row = row < rows ? row : rows - 1;
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+        mmd_dma4((op ? SB : SA) + row * (K / (32 / NW)) + 4 * NW * (int64_t)sk + 4 * w,
+                 __builtin_amdgcn_readfirstlane(lds_sc0 + (uint32_t)((((s & 1) * 2 + op) * NW + w) * 1024 + 256 * (wave % 4))));
+    }
+  };
+  auto batch1 = [&](int s) {
+#pragma unroll
+    for (int d = 0; d < 6; ++d) issue(s, d);
+    issue_scales(s);
+  };
+  auto batch2 = [&](int s) {
+    issue(s, 6);
+    issue(s, 7);
+  };
+  constexpr int INFL = 8 + NW; // a batch 1 and a batch 2
+
+  acc_t acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = acc_t{};
+
+  auto frag = [&](uint32_t base, int blk, int kb) -> v4i {
+    const int r = blk * 32 + lane % 32, g = 2 * kb + lane / 32;
+    return *(__attribute__((address_space(3))) const v4i *)(uintptr_t)(base + (uint32_t)((8 * r + (g ^ ((r >> 1) & 7))) * 16));
+  };
+  auto frag_kn = [&](uint32_t base, int blk, int kb) -> v4i {
+    typedef int v2i_ __attribute__((ext_vector_type(2)));
+    typedef short v4s_ __attribute__((ext_vector_type(4)));
+    const int q = lane / 16, j = lane % 16;
+    v4i f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v2i_ x;
+      if constexpr (ESZ == 1) {
+        const int kr = kb * 32 + 16 * (q / 2) + 8 * h + j / 2, g = blk * 2 + q % 2;
+        x = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (__attribute__((address_space(3))) v2i_ *)(uintptr_t)(base + (uint32_t)((kr * 16 + (g ^ kn_swz(kr))) * 16 + 8 * (j % 2))));
+      } else {
+        const int kr = kb * 16 + 8 * (q / 2) + 4 * h + j / 4, g = blk * 4 + 2 * (q % 2) + (j % 4) / 2;
+        x = __builtin_bit_cast(v2i_, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s_ *)(uintptr_t)(base + (uint32_t)((kr * 32 + (g ^ kn_swz(kr))) * 16 + 8 * (j % 2)))));
+      }
+      f[2 * h] = x.x;
+      f[2 * h + 1] = x.y;
+    }
+    return f;
+  };
+
+  v4i fa[4][2], fb[4][2];                       // [k-block][row / column block]
+  uint32_t sa_w[4][NW ? NW : 1], sb_w[2][NW ? NW : 1]; // scale words, shifted to this lane's k-half
+  auto read_a = [&](int s, int h) {
+    const uint32_t la = lds0 + (uint32_t)((s & 1) * 2 * MMD2_SLICE);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fa[kb][i] = frag(la, wm * 4 + 2 * h + i, kb);
+  };
+  auto read_b = [&](int s) {
+    const uint32_t lb = lds0 + (uint32_t)((s & 1) * 2 * MMD2_SLICE + MMD2_SLICE);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[kb][j] = BKN ? frag_kn(lb, wn * 2 + j, kb) : frag(lb, wn * 2 + j, kb);
+    if constexpr (MX) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sa_w[i][w] = lds_sc[s & 1][w][wm * 128 + i * 32 + lane % 32] >> (8 * (lane / 32));
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sb_w[j][w] = lds_sc[s & 1][NW + w][(wn * 2 + j) * 32 + lane % 32] >> (8 * (lane / 32));
+      }
+    }
+  };
+  auto mul = [&](auto hc) { // row half h: accumulator rows 2h, 2h + 1
+    constexpr int h = decltype(hc)::value;
+    if constexpr (MX && !FP4) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[2 * h + i][j] = Op::template run<0>(mx_cat(fa[0][i], fa[1][i]), mx_cat(fb[0][j], fb[1][j]), acc[2 * h + i][j],
+                                                  (int)sa_w[2 * h + i][0], (int)sb_w[j][0]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[2 * h + i][j] = Op::template run<2>(mx_cat(fa[2][i], fa[3][i]), mx_cat(fb[2][j], fb[3][j]), acc[2 * h + i][j],
+                                                  (int)sa_w[2 * h + i][0], (int)sb_w[j][0]);
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            acc_t &c = acc[2 * h + i][j];
+            if constexpr (!FP4) c = Op::run(fa[kb][i], fb[kb][j], c);
+            else
+              c = kb % 2 == 0 ? Op::template run<0>(mx_lo(fa[kb][i]), mx_lo(fb[kb][j]), c, (int)sa_w[2 * h + i][kb / 2], (int)sb_w[j][kb / 2])
+                              : Op::template run<2>(mx_lo(fa[kb][i]), mx_lo(fb[kb][j]), c, (int)sa_w[2 * h + i][kb / 2], (int)sb_w[j][kb / 2]);
+          }
+    }
+  };
+  auto end_phase = [&](bool even) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (even) mmd_wait_vm<INFL>();
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto run = [&](auto grp) { // group 0 computes in the even phases, group 1 in the odd ones
+    constexpr bool memEven = decltype(grp)::value == 1;
+    using h0 = std::integral_constant<int, 0>;
+    using h1 = std::integral_constant<int, 1>;
+#pragma unroll 1
+    for (int s = 0; s < nsteps; ++s) {
+      read_b(s);
+      read_a(s, 0);
+      batch2(s + 1);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      end_phase(memEven);
+      mul(h0{});
+      end_phase(!memEven);
+      read_a(s, 1);
+      batch1(s + 2);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      end_phase(memEven);
+      mul(h1{});
+      end_phase(!memEven);
+    }
+  };
+  batch1(0);
+  batch2(0);
+  batch1(1);
+  end_phase(true); // batch 1 of slice 0 has landed everywhere
+  if (wm == 0) {
+    run(std::integral_constant<int, 0>{});
+    asm volatile("s_barrier" ::: "memory"); // group 1's last turn
+  } else {
+    asm volatile("s_barrier" ::: "memory"); // group 0's first
+    run(std::integral_constant<int, 1>{});
+  }
+  mmd_wait_vm<0>();
+  __syncthreads();
+  mm_epilogue_lds<Epi, 2, 512, false>(acc, out, M, N, m0, n0, wm, wn, lane, P, &lds[0][0][0], (int)sizeof(lds));
 }
 
 // [R, C] row-major operand of ESZ-byte elements -> its [C, R] transpose, one
@@ -960,9 +1113,10 @@ __device__ __forceinline__ void mmad(const ElemT *A, const ElemT *B, typename Ep
                                      const Args &P) {
   static_assert(DMA == 0 || DMA == 4 || (!AT && BT), "the DMA rings 1 and 3 take K-contiguous A and B");
   static_assert(DMA == 0 || DMA == 1 || DMA == 3 || DMA == 4, "DMA mode");
-  if constexpr (DMA == 4) mmad_core_pp<MK, Epi, !BT, AT>(A, B, out, M, N, K, P);
+  if constexpr (DMA == 4 && AT) mmad_core_pp<MK, Epi, !BT, AT>(A, B, out, M, N, K, P);
+  else if constexpr (DMA == 4) mmad_core_alt<MK, Epi, true>(A, B, out, M, N, K, P);
   else if constexpr (mk_is_mx(MK)) static_assert(DMA == 4, "block-scaled kinds run on the [K, N] ring");
-  else if constexpr (DMA == 3) mmad_core_pp<MK, Epi, false>(A, B, out, M, N, K, P);
+  else if constexpr (DMA == 3) mmad_core_alt<MK, Epi, false>(A, B, out, M, N, K, P);
   else if constexpr (DMA == 1) mmad_core_dma<MK, Epi>(A, B, out, M, N, K, P);
   else mmad_core<MK, Epi, AT, BT>(A, B, out, M, N, K, P);
 }
@@ -975,7 +1129,7 @@ template <int MK, typename Epi, typename Args>
 __device__ __forceinline__ void mmad_mx(const uint8_t *A, const uint8_t *B, const uint8_t *SA, const uint8_t *SB,
                                         typename Epi::out_t *out, int64_t M, int64_t N, int64_t K, const Args &P) {
   static_assert(mk_is_mx(MK), "block-scaled kind");
-  mmad_core_pp<MK, Epi, true>(A, B, out, M, N, K, P, SA, SB);
+  mmad_core_alt<MK, Epi, true>(A, B, out, M, N, K, P, SA, SB);
 }
 
 } // namespace hf

@@ -1275,6 +1275,11 @@ def entries():
     for lay in ("nk", "kn"):
         e[f"tiles_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 1088, b_layout=lay), 7919)
         e[f"tiles_bf16_{lay}_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout=lay), 7919)
+    # the 256x256 ring with one to three slices of K, ragged tiles
+    e["ring_w8a8_nk_k128"] = g.w8a8_dequant(4000, 4016, 128)
+    e["ring_w8a8_kn_k256"] = g.w8a8_dequant(4000, 4016, 256, b_layout="kn")
+    e["ring_w8a8_nk_k384"] = g.w8a8_dequant(4000, 4016, 384)
+    e["ring_mx_e4m3_k128"] = g.matmul_mx(4000, 4016, 128, via="format")
     e["tiles_f16_kn_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout="kn", elem="f16"), 7919)
     e["tiles_mx_e4m3_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 1040, 640, via="format"), 7919)
     e["tiles_mx_e2m1_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 1040, 1280, fa="e2m1", fb="e2m1", via="format"), 7919)

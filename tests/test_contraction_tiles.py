@@ -12,6 +12,7 @@ import pytest
 
 import hfusion_mi355x as hf
 import group_catalog as cat
+from helpers import run_gpu
 from test_dynamic import _call
 from test_matmul_mx import TOL_FP4, fp4_case, fp4_products
 
@@ -106,3 +107,28 @@ def test_gpu_tiles_mx_fp4(gpu):
         out, = _call("tiles_mx_e2m1_rt", [a, b, sa, sb], gpu)
         mag, ref = fp4_products(ca, cb, sa, sb)
         assert np.all(np.abs(out.astype(np.float64) - ref) <= TOL_FP4 * mag + 1e-30)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,k,layout", [("ring_w8a8_nk_k128", 128, "nk"), ("ring_w8a8_kn_k256", 256, "kn"),
+                                           ("ring_w8a8_nk_k384", 384, "nk"), ("ring_mx_e4m3_k128", 128, "mx")])
+def test_gpu_ring_short_k(gpu, name, k, layout):
+    """The alternating wave groups with fewer slices than they keep in
+    flight: re-read slices must not reach a result."""
+    print(f"[case] {name}", flush=True)
+    rng, m, n = np.random.default_rng(81), 4000, 4016
+    if layout == "mx":
+        # small whole numbers in e4m3 (0 .. 7 and -7 .. 0) with unit scales: exact sums
+        code = np.array([0x00, 0x38, 0x40, 0x44, 0x48, 0x4A, 0x4C, 0x4E], np.uint8)
+        ia, ib = rng.integers(-7, 8, (m, k)), rng.integers(-7, 8, (k, n))
+        enc = lambda v: (code[np.abs(v)] | np.where(v < 0, 0x80, 0).astype(np.uint8))
+        sc = [np.full((r, k // 32), 127, np.uint8) for r in (m, n)]
+        out, = run_gpu(name, [enc(ia), enc(ib)] + sc, gpu)
+        assert np.array_equal(out.astype(np.float64), ia.astype(np.float64) @ ib.astype(np.float64))
+        return
+    a = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    b = rng.integers(-127, 128, (n, k) if layout == "nk" else (k, n), dtype=np.int8)
+    c = a.astype(np.float64) @ (b.T if layout == "nk" else b).astype(np.float64)
+    st, sc = rng.uniform(0.001, 0.02, m).astype(np.float32), rng.uniform(0.001, 0.02, n).astype(np.float32)
+    out, = run_gpu(name, [a, b, st, sc, np.zeros((m, n), np.uint16)], gpu)
+    assert np.array_equal(out.view(np.uint16), I.f32_to_bf16_bits((c.astype(np.float32) * st[:, None]) * sc[None, :]))
