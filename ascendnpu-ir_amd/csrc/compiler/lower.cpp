@@ -2424,16 +2424,19 @@ constexpr int MK_BF16_CODE = 1; // hf::MK_BF16
 // W8A8 and bf16 alike at N = 4096): `one` workgroup on a CU, a `second` beside
 // it, each one `more` (0: a CU holds one, the next wait).  Both sides of the
 // lines they draw, W8A8 at N = K = 4096: M = 64: 6.1 us (32x32) against 10.1
-// (64x64); M = 128: 8.5 (64x32) against 10.7 (64x64); M = 333: 12.8 (64x64)
-// against 13.5 (128x64); M = 1024: 22.6 (128x128) against 23.8 (128x64) and
+// (64x64); M = 128: 8.5 (64x32) against 10.7 (64x64); M = 200: 10.9 (64x64, two
+// slices a stage) against 11.8 (one); M = 333: 13.5 (64x64, one) against 14.6
+// (128x64, two) and 15.3 (128x64, one), and of a [K, N] B 14.7 (64x128, two)
+// against 16.0 (64x64, one); M = 1024: 22.6 (128x128) against 23.8 (128x64) and
 // 31.6 (256x128); M = 2048: 40.7 (256x128) against 46.1 (128x128 and
 // 256x256); block-scaled fp8, M = 2048: 56.6 (256x256) against 60.9 (128x128).
 struct ContractionTile {
   char kind;           // 's' mmad_skinny, 't' mmad_tile, 'r' the 256x256 ring kernels of hf_mmad.h
-  int tm, tn, a, b, s; // 's': a waves; 't': a x b waves, s ring stages
+  int tm, tn, a, b, s; // 's': a waves; 't': a x b waves per slice of K, s ring stages
   double one, second, more;
-  bool operator==(const ContractionTile &o) const { return kind == o.kind && tm == o.tm && tn == o.tn; }
-  int threads() const { return kind == 'r' ? 512 : 64 * a * (kind == 's' ? 1 : b); }
+  int kg = 1;          // 't': slices of K (and groups of a x b waves) per stage
+  bool operator==(const ContractionTile &o) const { return kind == o.kind && tm == o.tm && tn == o.tn && kg == o.kg; }
+  int threads() const { return kind == 'r' ? 512 : 64 * kg * a * (kind == 's' ? 1 : b); }
   // workgroups of one row of tiles (in eighths: an XCD each)
   int64_t blocksPerRow(int64_t N) const {
     const int64_t t = (N + tn - 1) / tn;
@@ -2444,14 +2447,16 @@ const ContractionTile kRing256 = {'r', 256, 256, 0, 0, 0, 60, 0, 0};
 
 ContractionTile pickTile(int64_t M, int64_t N, int64_t Kb, bool bT, int mk) {
   static const std::vector<ContractionTile> nk = {
-      {'s', 16, 16, 8, 0, 0, 2.4, 0, 0},   {'s', 32, 16, 8, 0, 0, 2.8, 0, 0},    {'s', 32, 32, 8, 0, 0, 3.8, 0, 0},
-      {'s', 64, 32, 4, 0, 0, 6.2, 0, 0},   {'t', 64, 64, 2, 2, 3, 8.4, 4, 7.5},  {'t', 128, 64, 4, 2, 3, 12, 10, 14},
-      {'t', 128, 128, 4, 4, 3, 20.5, 0, 0}, {'t', 256, 128, 4, 2, 3, 35, 0, 0},  kRing256};
+      {'s', 16, 16, 8, 0, 0, 2.4, 0, 0},        {'s', 32, 16, 8, 0, 0, 2.8, 0, 0},      {'s', 32, 32, 8, 0, 0, 3.8, 0, 0},
+      {'s', 64, 32, 4, 0, 0, 6.2, 0, 0},        {'t', 64, 64, 2, 2, 3, 7.4, 0, 0, 2},   {'t', 64, 64, 2, 2, 3, 8.8, 5.5, 7.5},
+      {'t', 128, 64, 4, 2, 3, 12, 10, 14},      {'t', 128, 128, 4, 4, 3, 20.5, 0, 0},     {'t', 256, 128, 4, 2, 3, 35, 0, 0},
+      kRing256};
   // B [K, N]: short pieces of every k-row make the narrow tiles slower
   static const std::vector<ContractionTile> kn = {
-      {'s', 16, 16, 8, 0, 0, 6.9, 0, 0},  {'s', 32, 16, 8, 0, 0, 7.4, 0, 0},       {'s', 32, 32, 8, 0, 0, 8.6, 0, 0},
-      {'t', 32, 64, 1, 2, 4, 9, 5, 6},    {'t', 64, 64, 2, 2, 3, 10.2, 6.5, 8}, {'t', 128, 64, 4, 2, 3, 12.6, 10, 14.5},
-      {'t', 128, 128, 4, 4, 3, 21, 0, 0}, {'t', 256, 128, 4, 2, 3, 36.5, 0, 0},  kRing256};
+      {'s', 16, 16, 8, 0, 0, 6.9, 0, 0},        {'s', 32, 16, 8, 0, 0, 7.4, 0, 0},      {'s', 32, 32, 8, 0, 0, 8.6, 0, 0},
+      {'t', 32, 64, 1, 2, 4, 9, 5, 6},          {'t', 64, 64, 2, 2, 3, 9.6, 0, 0, 2},   {'t', 64, 64, 2, 2, 3, 10.9, 6.5, 8},
+      {'t', 64, 128, 2, 4, 3, 12.2, 0, 0, 2},   {'t', 128, 64, 4, 2, 3, 13, 13, 14.5},  {'t', 128, 128, 4, 4, 3, 19.5, 0, 0},
+      {'t', 256, 128, 4, 2, 3, 36.5, 0, 0},     kRing256};
   // block-scaled (the scaled instruction takes wider wave tiles)
   static const std::vector<ContractionTile> fp8 = {
       {'t', 32, 64, 1, 2, 4, 8, 0, 0}, {'t', 64, 64, 2, 2, 3, 12, 0, 0}, {'t', 64, 128, 2, 2, 3, 15.3, 0, 0},
@@ -2466,6 +2471,7 @@ ContractionTile pickTile(int64_t M, int64_t N, int64_t Kb, bool bT, int mk) {
     // (the 256x256 ring of 64-byte slices took 650 us at M = 3000, N = 4096,
     // K = 4032, where the 256x128 tiles take 76)
     if (t.kind == 'r' && Kb % 128 != 0) continue;
+    if (t.kg > 1 && Kb < 1024) continue; // (the groups' sums cost more than they save)
     const double n = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn) / 256;
     double cost = n <= 1 ? t.one : !t.second ? t.one * std::ceil(n) : n <= 2 ? t.one + t.second * (n - 1) : t.one + t.second + t.more * (n - 2);
     // the ring kernels leave the other CUs' power and L2 to the busy ones:
@@ -2743,7 +2749,10 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
     k << "  hf::" << (mx ? "mmad_mx<" : t.kind == 's' ? "mmad_skinny<" : "mmad_tile<") << mk << ", " << kname << "_epi, "
       << (mx ? "" : bT ? "false, " : "true, ");
     if (t.kind == 's') k << t.tm / 16 << ", " << t.tn / 16 << ", " << t.a;
-    else k << t.tm << ", " << t.tn << ", " << t.a << ", " << t.b << ", " << t.s;
+    else {
+      k << t.tm << ", " << t.tn << ", " << t.a << ", " << t.b << ", " << t.s;
+      if (!mx) k << ", " << t.kg;
+    }
     k << ">((const " << tt << "*)p" << a->argIdx << ", (const " << tt << "*)p" << b->argIdx;
     if (mx) k << ", (const uint8_t*)p" << sa->argIdx << ", (const uint8_t*)p" << sb->argIdx;
     k << ", (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
@@ -2755,7 +2764,7 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
     for (int64_t m = 16; m <= 16384; m += m < 64 ? 16 : 64) {
       const ContractionTile t = pickTile(m, N, K * esz, bT, mk);
       if (t.kind == 'r') break;
-      const std::string nm = kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn);
+      const std::string nm = kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn) + (t.kg > 1 ? "k" + std::to_string(t.kg) : "");
       if (!p.alts.empty() && p.alts.back().name == nm) { p.alts.back().maxRows = m; continue; }
       if (std::find(emitted.begin(), emitted.end(), t) == emitted.end()) {
         emitted.push_back(t);

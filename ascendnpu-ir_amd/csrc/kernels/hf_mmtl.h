@@ -29,12 +29,28 @@ template <int S, int CNT> __device__ __forceinline__ void mmt_wait_ahead(int ahe
   }
 }
 
+// A wave-uniform pointer in scalar registers, as mmd_dma16_off's base has to be:
+// the compiler selects between two of them in vector registers at times.
+__device__ __forceinline__ const char *mmt_uniform(const char *p) {
+  const uint64_t u = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return reinterpret_cast<const char *>((uint64_t)hi << 32 | lo);
+}
+
 // One workgroup of WM x WN waves per TM x TN tile of C; wave (wm, wn) holds
 // TM / WM rows and TN / WN columns as 32x32 matrix-core tiles.  K advances in
 // slices of 128 bytes (the last may be half) through a ring of S stages:
 // step s waits for its slice, passes the one barrier of the step (which also
 // says that everyone has read slice s - 1), refills the slot of slice s - 1
 // with slice s + S - 1 and multiplies slice s.
+// KG > 1: a stage holds KG slices and KG groups of WM x WN waves multiply one
+// each, so that there are as many times fewer barriers and waits, and more
+// waves to fill them; the groups' partial sums meet in LDS at the end.  It
+// pays while a CU has one tile (N = K = 4096, 64x64 KG 1 -> 2 at M = 200: W8A8
+// 11.8 -> 10.9 us, bf16 20.6 -> 17.5) and, of a [K, N] B, against the two
+// resident narrower tiles too (M = 333: W8A8 64x64 KG 1 -> 64x128 KG 2 16.0 ->
+// 14.8 us, bf16 27 -> 24); of an [N, K] B those are as fast (13.5 against 14.6,
+// 23.8 against 23.6).
 // Operands as in hf_mmad.h: A [M, K] row-major; B [N, K] row-major, or
 // [K, N] with BKN.  Row-major slices: granule g (16 bytes) of row r at
 // position g ^ ((r >> 1) & 7).  K-major slices: k-rows of TN columns as they
@@ -43,7 +59,7 @@ template <int S, int CNT> __device__ __forceinline__ void mmt_wait_ahead(int ahe
 // groups and leaves the granule bits apart that tell those groups.
 // Block-scaled kinds: SA [M, K/32], SB [N, K/32] e8m0 bytes ride the ring,
 // 4 (fp4: 8) bytes per row and stage.
-template <int MK, typename Epi, bool BKN, int TM, int TN, int WM, int WN, int S, typename ElemT, typename Args>
+template <int MK, typename Epi, bool BKN, int TM, int TN, int WM, int WN, int S, int KG = 1, typename ElemT, typename Args>
 __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const ElemT *__restrict__ B,
                                           typename Epi::out_t *__restrict__ out, int64_t M, int64_t N, int64_t K, const Args &P,
                                           const uint8_t *__restrict__ SA = nullptr, const uint8_t *__restrict__ SB = nullptr) {
@@ -53,8 +69,10 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
   using Op = typename std::conditional<MX, MfmaMx<(MX ? MK : MK_MX)>, MfmaOp<(MX ? MK_I8 : MK)>>::type;
   using acc_t = typename Op::acc_t;
   using O = typename Epi::out_t;
-  constexpr int ESZ = sizeof(ElemT), NW = WM * WN, IT = TM / WM / 32, JT = TN / WN / 32;
-  constexpr int SLOT = (TM + TN) * 128, DA = TM / 8, DT = (TM + TN) / 8; // bytes, DMA instructions of A, of both
+  constexpr int ESZ = sizeof(ElemT), NWG = WM * WN, NW = NWG * KG, IT = TM / WM / 32, JT = TN / WN / 32;
+  constexpr int SL = (TM + TN) * 128, SLOT = KG * SL;                         // bytes of a slice, of a stage
+  constexpr int DA = TM / 8, DS = (TM + TN) / 8, DT = KG * DS;                // DMA instructions: A, slice, stage
+  static_assert(!MX || KG == 1, "block-scaled kinds: one slice per stage");
   static_assert(DT % NW == 0, "every wave issues as many DMA instructions");
   constexpr int DW = DT / NW;                                               // per wave and stage
   constexpr int SCE = (TM + TN + 63) / 64 * 64;                               // scale entries: A rows, B columns, padding
@@ -73,8 +91,8 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
   const int64_t m0 = (int64_t)ti * TM, n0 = (int64_t)tj * TN;
   const int64_t Kb = K * ESZ;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
-  const int wm = wave / WN, wn = wave % WN;
-  const int nsteps = (int)((Kb + 127) / 128);
+  const int kg = wave / NWG, wm = wave % NWG / WN, wn = wave % WN; // K group, place in the tile
+  const int nslices = (int)((Kb + 127) / 128), nsteps = (nslices + KG - 1) / KG;
   const bool half = Kb % 128 != 0;
   const char *Ab = reinterpret_cast<const char *>(A), *Bb = reinterpret_cast<const char *>(B);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&lds[0];
@@ -93,7 +111,7 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
   uint32_t back[DW];
 #pragma unroll
   for (int d = 0; d < DW; ++d) {
-    const int x = wave + d * NW; // instruction of the stage (A first): whole operands per d where NW divides them
+    const int x = KG == 1 ? wave + d * NW : (wave + d * NW) % DS; // instruction of its slice (A first)
     const bool isA = x < DA;
     const int64_t rows = isA ? M : N, row0 = isA ? m0 : n0;
     if (isA || !BKN) {
@@ -109,16 +127,27 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
       back[d] = kr >= 64 / ESZ ? (uint32_t)(64 * N) : 0u;
     }
   }
-  const char *const a0 = Ab + m0 * Kb, *const b0 = BKN ? Bb : Bb + n0 * Kb;
-  const int64_t bstep = BKN ? 128 * N : 128;
-  auto issue = [&](int s) {
+  // each instruction's slice of the stage in flight next, its address and step
+  const char *src[DW];
+  int64_t step[DW];
+  int next[DW];
+#pragma unroll
+  for (int d = 0; d < DW; ++d) {
+    const int y = wave + d * NW, x = KG == 1 ? y : y % DS;
+    next[d] = KG == 1 ? 0 : y / DS;
+    step[d] = x < DA || !BKN ? 128 : 128 * N;
+    if (next[d] >= nslices) next[d] = nslices - 1; // (a slice past the end: the last again, not multiplied)
+    src[d] = mmt_uniform((x < DA ? Ab + m0 * Kb : BKN ? Bb : Bb + n0 * Kb) + next[d] * step[d]);
+  }
+  auto issue = [&](int s) { // s = 0, 1, 2, ...
     const uint32_t slot = lds0 + (uint32_t)(s % S * SLOT);
-    const bool tail = half && s == nsteps - 1;
 #pragma unroll
     for (int d = 0; d < DW; ++d) {
-      const int x = wave + d * NW;
-      const char *base = x < DA ? a0 + (int64_t)s * 128 : b0 + (int64_t)s * bstep;
-      mmd_dma16_off(base, tail ? dofs[d] - back[d] : dofs[d], __builtin_amdgcn_readfirstlane(slot + (uint32_t)(x * 1024)));
+      mmd_dma16_off(src[d], half && next[d] == nslices - 1 ? dofs[d] - back[d] : dofs[d],
+                    __builtin_amdgcn_readfirstlane(slot + (uint32_t)((wave + d * NW) * 1024)));
+      const int adv = KG == 1 || next[d] + KG < nslices ? KG : nslices - 1 - next[d];
+      src[d] += adv * step[d];
+      next[d] += adv;
     }
     if constexpr (MX) {
 #pragma unroll
@@ -180,8 +209,9 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
     mmt_wait_ahead<S - 1, DPS>(nsteps - 1 - s);
     __syncthreads();
     if (s + S - 1 < nsteps) issue(s + S - 1);
-    const uint32_t slot = lds0 + (uint32_t)(s % S * SLOT);
-    const bool tail = half && s == nsteps - 1;
+    const uint32_t slot = lds0 + (uint32_t)(s % S * SLOT + kg * SL);
+    const bool tail = half && s * KG + kg == nslices - 1;
+    if (KG > 1 && s * KG + kg >= nslices) continue; // (no barrier follows in the loop body)
     uint32_t sa[IT][NWD], sb[JT][NWD];
     if constexpr (MX) {
       // this lane's scale words: byte 2 h (fp4: byte 2 kk of word h) is the
@@ -237,6 +267,27 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
     }
   }
 
+  if constexpr (KG > 1) {
+    // the other K groups' partial sums through the ring, added in K order
+    static_assert((KG - 1) * TM * TN * 4 <= LDSB, "partial sums");
+    acc_t *red = reinterpret_cast<acc_t *>(lds);
+    __syncthreads();
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+#pragma unroll
+        for (int j = 0; j < JT; ++j) red[(((kg - 1) * NWG + wm * WN + wn) * IT * JT + i * JT + j) * 64 + lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+#pragma unroll
+          for (int j = 0; j < JT; ++j) acc[i][j] += red[((q * NWG + wm * WN + wn) * IT * JT + i * JT + j) * 64 + lane];
+    }
+  }
   // outputs through the (now free) ring into row-major 16-byte stores;
   // accumulator register r of a 32x32 tile is row 8 (r / 4) + 4 (lane / 32) +
   // r % 4, column lane % 32.  PASS rows at a time when the tile does not fit.
@@ -246,7 +297,7 @@ __device__ __forceinline__ void mmad_tile(const ElemT *__restrict__ A, const Ele
 #pragma unroll 1
   for (int h = 0; h < NP; ++h) {
     __syncthreads();
-    if (NP == 1 || wm / (WM / NP) == h) {
+    if (kg == 0 && (NP == 1 || wm / (WM / NP) == h)) {
 #pragma unroll
       for (int i = 0; i < IT; ++i) {
         typename Epi::row_t rv[16];

@@ -1275,6 +1275,8 @@ def entries():
     for lay in ("nk", "kn"):
         e[f"tiles_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 1088, b_layout=lay), 7919)
         e[f"tiles_bf16_{lay}_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout=lay), 7919)
+        # ... and the ones of two slices a stage, with 8.5 slices
+        e[f"tiles_bf16_{lay}_k544_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 544, b_layout=lay), 7919)
     # the 256x256 ring with one to three slices of K, ragged tiles
     e["ring_w8a8_nk_k128"] = g.w8a8_dequant(4000, 4016, 128)
     e["ring_w8a8_kn_k256"] = g.w8a8_dequant(4000, 4016, 256, b_layout="kn")

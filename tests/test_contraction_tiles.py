@@ -30,7 +30,7 @@ def test_alternatives_by_row_count():
         rows = [int(a[1]) for a in alts]
         assert rows == sorted(set(rows)) and len(alts) >= 5
         for kern, top, rb, rc, threads in alts:
-            tm, tn = (int(v) for v in kern.rsplit("_", 1)[1].split("x"))
+            tm, tn = (int(v) for v in kern.rsplit("_", 1)[1].split("k")[0].split("x"))
             assert int(rb) == tm and int(rc) == (-(-N // tn) + 7) // 8 * 8 and int(threads) <= 1024
             blk = hf.compile(hf.groups.w8a8_dequant(int(top), N, k, b_layout=layout), options="emit=hip").blocks[0]
             assert f"{tm}x{tn} tiles" in blk["variant"]
@@ -56,6 +56,24 @@ def test_gpu_tiles_w8a8(gpu, layout):
         out, = _call(f"tiles_w8a8_{layout}_rt", [a, b, st, sc, np.zeros((m, N), np.uint16)], gpu)
         ref = I.f32_to_bf16_bits((c.astype(np.float32) * st[:, None]) * sc[None, :])
         assert np.array_equal(out.view(np.uint16), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [150, 257, 960, 1100, 1791])
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+def test_gpu_tiles_two_slices(gpu, layout, m):
+    """Two slices of K a stage: 8.5 slices, the last stage of the second wave
+    group past the end; whole-number values, exact sums."""
+    print(f"[case] two slices {layout} M={m}", flush=True)
+    rng, k = np.random.default_rng(79), 544
+    fa, fb = rng.integers(-3, 4, (m, k)).astype(np.float32), rng.integers(-3, 4, (N, k) if layout == "nk" else (k, N)).astype(np.float32)
+    out, = _call(f"tiles_bf16_{layout}_k544_rt", [I.f32_to_bf16_bits(fa), I.f32_to_bf16_bits(fb), np.zeros((m, N), np.uint16)], gpu)
+    # (|sum| <= 9 * 544 < 2^24: every order of adding gives it, rounded once)
+    assert np.array_equal(out.view(np.uint16), I.f32_to_bf16_bits(fa @ (fb.T if layout == "nk" else fb)))
+    a, b, c = _mm(rng, m, 1088, layout)
+    st, sc = rng.uniform(0.001, 0.02, m).astype(np.float32), rng.uniform(0.001, 0.02, N).astype(np.float32)
+    out, = _call(f"tiles_w8a8_{layout}_rt", [a, b, st, sc, np.zeros((m, N), np.uint16)], gpu)
+    assert np.array_equal(out.view(np.uint16), I.f32_to_bf16_bits((c.astype(np.float32) * st[:, None]) * sc[None, :]))
 
 
 @pytest.mark.gpu
