@@ -9,11 +9,13 @@
 //   * f16 x f16 -> fp32 with v_mfma_f32_32x32x16_f16.
 // One 256x256 macro-tile per workgroup of 4 waves (2 x 2, 128x128 each =
 // 4 x 4 MFMA tiles of 32x32), K advanced 64 bytes at a time.
-//   * DMA path (B [N, K], K spanning a multiple of 64 bytes): a 4-slot LDS
-//     ring filled by global_load_lds_dwordx4 four steps ahead of the MFMAs,
+//   * DMA path, 64-byte slices (both operands K-contiguous): a 4-slot LDS ring
+//     filled by global_load_lds_dwordx4 four steps ahead of the MFMAs,
 //     fragments double-buffered in registers (one barrier per step);
-//   * register path (the rest): a double-buffered LDS stage with register
-//     prefetch of the next K slice.
+//   * register path (K not a multiple of 64 bytes): a double-buffered LDS
+//     stage with register prefetch of the next K slice;
+//   * DMA paths, 128-byte slices, 8 waves: mmad_core_alt, mmad_core_pp below.
+// Smaller tiles: hf_mmsk.h, hf_mmtl.h.
 // Macro-tiles are numbered so that the workgroups the dispatcher sends to one
 // XCD (blockIdx % 8) cover a compact 2-D block of C and share A/B panels in
 // that XCD's L2.  The epilogue functor receives the raw accumulator and the
@@ -541,13 +543,12 @@ constexpr int MMD2_SLICE = 256 * 128;
 // k-row k0 + j/2 at column c0 + 8 (j % 2) gives lane i the column c0 + i at
 // k-rows k0 .. k0+7 -- eight consecutive k-bytes of one column, as the matrix
 // core takes them.
-// AKM: A is [K, M] (hivm a_transpose), staged and read exactly as a [K, N] B
-// (its M columns in place of N).
-template <int MK, typename Epi, bool BKN, bool AKM = false, typename ElemT, typename Args>
+// A is [K, M] (hivm a_transpose), staged and read exactly as a [K, N] B (its M
+// columns in place of N); a row-major A goes to mmad_core_alt.
+template <int MK, typename Epi, bool BKN, typename ElemT, typename Args>
 __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restrict__ B, typename Epi::out_t *__restrict__ out,
                              int64_t M, int64_t N, int64_t K, const Args &P) {
-  static_assert(!(BKN || AKM) || ((MK == MK_I8 && sizeof(ElemT) == 1) ||
-                                  ((MK == MK_BF16 || MK == MK_F16) && sizeof(ElemT) == 2)),
+  static_assert((MK == MK_I8 && sizeof(ElemT) == 1) || ((MK == MK_BF16 || MK == MK_F16) && sizeof(ElemT) == 2),
                 "the K-major operand path takes bytes or 16-bit floats");
   using Op = MfmaOp<MK>;
   using acc_t = typename Op::acc_t;
@@ -590,7 +591,7 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
 #pragma unroll
   for (int d = 0; d < 8; ++d) {
     const int blk = wave * 4 + (d & 3);
-    const bool kmaj = d >= 4 ? BKN : AKM; // this operand is stored [K, columns]
+    const bool kmaj = d < 4 || BKN; // this operand is stored [K, columns]
     if (kmaj) {
       const int64_t cols = d >= 4 ? N : M, c0 = d >= 4 ? n0 : m0;
       if constexpr (ESZ == 1) {
@@ -609,14 +610,12 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
     } else {
       const int r = 8 * blk + lane / 8;
       const int g = (lane % 8) ^ ((r >> 1) & 7);
-      const int64_t rows = d < 4 ? M : N, row0 = d < 4 ? m0 : n0;
-      int64_t row = row0 + r;
-      row = row < rows ? row : rows - 1;
-      dofs[d] = (uint32_t)((row - row0) * Kb + g * 16);
+      const int64_t row = n0 + r < N ? n0 + r : N - 1;
+      dofs[d] = (uint32_t)((row - n0) * Kb + g * 16);
     }
   }
-  const char *const dbase[2] = {AKM ? Ab : Ab + m0 * Kb, BKN ? Bb : Bb + n0 * Kb};
-  const int64_t dstride[2] = {AKM ? 128 * M : 128, BKN ? 128 * N : 128};
+  const char *const dbase[2] = {Ab, BKN ? Bb : Bb + n0 * Kb};
+  const int64_t dstride[2] = {128 * M, BKN ? 128 * N : 128};
   auto issue_one = [&](int s, int slot, int d) {
     const uint32_t st = lds0 + (uint32_t)(slot * 2 * MMD2_SLICE) + (d < 4 ? 0u : (uint32_t)MMD2_SLICE) +
                         (uint32_t)((wave * 4 + (d & 3)) * 1024);
@@ -684,8 +683,7 @@ __device__ void mmad_core_pp(const ElemT *__restrict__ A, const ElemT *__restric
     for (int q = 0; q < 2; ++q) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        f[q][i] = !AKM ? frag(la, wm * 4 + i, 4 * h + 2 * q + lane / 32)
-                  : ESZ == 1 ? frag_kn(la, wm * 4 + i, 2 * h + q) : frag_kn16(la, wm * 4 + i, 2 * h + q);
+        f[q][i] = ESZ == 1 ? frag_kn(la, wm * 4 + i, 2 * h + q) : frag_kn16(la, wm * 4 + i, 2 * h + q);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         f[q][4 + j] = !BKN ? frag(lb, wn * 2 + j, 4 * h + 2 * q + lane / 32)
@@ -1113,7 +1111,7 @@ __device__ __forceinline__ void mmad(const ElemT *A, const ElemT *B, typename Ep
                                      const Args &P) {
   static_assert(DMA == 0 || DMA == 4 || (!AT && BT), "the DMA rings 1 and 3 take K-contiguous A and B");
   static_assert(DMA == 0 || DMA == 1 || DMA == 3 || DMA == 4, "DMA mode");
-  if constexpr (DMA == 4 && AT) mmad_core_pp<MK, Epi, !BT, AT>(A, B, out, M, N, K, P);
+  if constexpr (DMA == 4 && AT) mmad_core_pp<MK, Epi, !BT>(A, B, out, M, N, K, P);
   else if constexpr (DMA == 4) mmad_core_alt<MK, Epi, true>(A, B, out, M, N, K, P);
   else if constexpr (mk_is_mx(MK)) static_assert(DMA == 4, "block-scaled kinds run on the [K, N] ring");
   else if constexpr (DMA == 3) mmad_core_alt<MK, Epi, false>(A, B, out, M, N, K, P);
