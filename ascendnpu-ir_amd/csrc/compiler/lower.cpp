@@ -2345,8 +2345,10 @@ KernelPlan lowerReduceWithIndex(Analysis &A, const std::string &kname) {
   p.source = k.str();
   p.grid[0] = (unsigned)(R * segs);
   p.block[0] = BLOCK;
-  // workspace: per-segment partial records + one arrival counter per row
-  p.workspaceBytes = (uint64_t)(R * segs * 8 + R * 128 + 256);
+  // workspace: per-segment partial records + one arrival counter per row,
+  // 128 bytes apart (whole rows per workgroup leave no record and count
+  // nothing: their workspace does not grow with the rows)
+  p.workspaceBytes = segs == 1 ? 256 : (uint64_t)(R * segs * 8 + R * 128 + 256);
   p.workspaceZeroInit = true;
   return p;
 }

@@ -1179,6 +1179,7 @@ def entries():
     e["argmax_i64"] = g.argmax(8, 4096, index_type="i64")
     e["argmin_ragged"] = g.argmax(9, 5001, kind="min")
     e["argmax_row"] = g.argmax(1, 2100004)  # 512 segments
+    e["argmax_many_rows"] = g.argmax(40000, 100)
     e["argmax_tall"] = g.argmax(2048, 33797)
     e["w8a8_512"] = g.w8a8_dequant(512, 512, 512)
     e["w8a8_ragged"] = g.w8a8_dequant(300, 200, 160)

@@ -304,3 +304,16 @@ def test_external_declarations_are_skipped(decl, tmp_path):
     rc, err, prefix = emit(ir, tmp_path)
     assert rc == 0, err
     assert [b["func"] for b in hf.parse_manifest(prefix + ".manifest")] == ["vec_add"]
+
+
+def test_argmax_workspace_does_not_grow_with_whole_rows():
+    """Rows that workgroups take whole need no records and no counters, so a
+    group of any row count stays within the scratch of launches that may not
+    allocate; split rows keep one record a segment and one counter a row."""
+    scratch = 4 << 20
+    for rows, cols in ((256, 152064), (40000, 100), (200000, 16)):
+        b = hf.compile(hf.groups.argmax(rows, cols), options="emit=hip").blocks[0]
+        assert b["grid"][0] == rows and 0 < b["workspace"] <= 256
+    for rows, cols in ((255, 152064), (1, 2100004)):
+        b = hf.compile(hf.groups.argmax(rows, cols), options="emit=hip").blocks[0]
+        assert b["grid"][0] > rows and b["grid"][0] * 8 + rows * 128 <= b["workspace"] <= scratch

@@ -54,6 +54,16 @@ def test_noalloc_argreduce_matches(gpu, big, small):
         _same(got, ref)
 
 
+def test_noalloc_argreduce_many_rows(gpu):
+    """More rows than the scratch could hold arrival counters for: whole rows
+    per workgroup need none."""
+    note("noalloc argmax_many_rows 40000x100")
+    x = np.random.default_rng(41).standard_normal((40000, 100)).astype(np.float32)
+    args = [x, np.zeros(40000, np.float32), np.zeros(40000, np.int32)]
+    got, _ = _run("argmax_many_rows", args, gpu, noalloc=True)
+    assert np.array_equal(got[0], x.max(axis=1)) and np.array_equal(got[1], x.argmax(axis=1))
+
+
 def test_noalloc_histogram_matches(gpu):
     native_bytes = native.hfr().hfr_scratch_bytes()
     for name in ("hist_mask_i64", "hist_i8_wrap"):  # the second is the smaller input
