@@ -1388,7 +1388,9 @@ struct RowEmitter {
     int64_t nch = (C + span - 1) / span;
     EPL = (int)(nch * VEC);
     masked = (C % span) != 0;
-    if (EPL * RPW > 256)
+    // (a serial-order row is as wide as 4 resident rows of a wave allow,
+    // whatever the row count: one row of 256 elements a lane spills)
+    if (EPL * (needOrdered ? 4 : RPW) > 256)
       throw CompileError("row of " + std::to_string(C) + " elements does not fit one row group");
     if (needOrdered) {
       int jpc = std::max<int64_t>(1, 512 / span);

@@ -317,3 +317,18 @@ def test_argmax_workspace_does_not_grow_with_whole_rows():
     for rows, cols in ((255, 152064), (1, 2100004)):
         b = hf.compile(hf.groups.argmax(rows, cols), options="emit=hip").blocks[0]
         assert b["grid"][0] > rows and b["grid"][0] * 8 + rows * 128 <= b["workspace"] <= scratch
+
+
+def test_serial_order_rows_have_one_widest_row(tmp_path):
+    """A row whose float sum is folded in serial order holds at most 4096
+    elements, at every row count, static or given at launch."""
+    for rows in (1, 100, 2048, 2049, 4096, 4097, 8192):
+        for cols in (4097, 5000, 8192, 16384):
+            rc, err, _ = emit(hf.groups.rmsnorm_quant(rows, cols), tmp_path)
+            assert rc == -2 and f"row of {cols} elements does not fit one row group" in err, (rows, cols, err)
+        assert emit(hf.groups.rmsnorm_quant(rows, 4095), tmp_path)[0] == 0
+    ir = hf.groups.with_dynamic_rows(hf.groups.rmsnorm_quant(7919, 8192), 7919)
+    assert "does not fit one row group" in emit(ir, tmp_path, options="dyn=runtime")[1]
+    # other float sums of wide rows are folded in tree order, unless asked for
+    assert emit(hf.groups.safe_softmax(100, 8192), tmp_path)[0] == 0
+    assert "does not fit one row group" in emit(hf.groups.safe_softmax(100, 8192), tmp_path, options="ordered_fp_sums=1")[1]
