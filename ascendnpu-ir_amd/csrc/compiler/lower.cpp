@@ -1363,6 +1363,19 @@ struct RowEmitter {
     // (a row length that is no multiple of VEC keeps the width: rows then
     // start on any element and the last chunk is masked.  Softmax, 4096 rows
     // of 32767: 181 -> 147 us, of 5003 33.9 -> 25.9)
+    if (needOrdered && rowsHint > 4096) {
+      // with 32 rows a block it is the lanes' work that counts, and a narrow
+      // row's padding to 64 VEC columns (127 columns: 128 or 256) is work and
+      // LDS: there the width that divides the row.  f32 softmax, 16384 rows,
+      // full against dividing width: of 127 10.1 and 5.9 us, of 603 21.0 and
+      // 19.4, of 701 22.5 and 21.6, but 20000 of 702 31.4 and 33.1, 16384 of 2001
+      // 54 and 58.  Rows of 16-bit elements on 8-byte boundaries: norm +
+      // quant, 16384 rows of 772 26.5 and 21.9, of 2412 48.6 and 44.2, 20000 of
+      // 3204 84.4 and 79.3, but 16384 of 3604 65 and 68
+      int div = VEC;
+      while (div > 1 && C % div) div /= 2;
+      if (C <= 160 * VEC || (div >= 4 && C <= 3328)) VEC = div;
+    }
     if (needOrdered) {
       // one wave per row group of up to 4 rows, up to 8 waves: at most 32 rows
       // per block with a single serial chain lane per row in wave 0 (2 waves
@@ -1719,7 +1732,7 @@ struct RowEmitter {
         storeLoop("ex", "    ");
         const std::string rcp = q.qRcpRow ? q.qRcp + "[rr]" : q.qRcp;
         body << "  } else {\n#pragma unroll\n    for (int rr = 0; rr < RPW; ++rr)\n#pragma unroll\n"
-             << "      for (int j = 0; j < EPL / VEC; ++j) {\n        uint32_t st_[VEC / 4];\n#pragma unroll\n"
+             << "      for (int j = 0; j < EPL / VEC; ++j) {\n        uint32_t st_[(VEC + 3) / 4];\n#pragma unroll\n"
              << "        for (int w = 0; w < VEC / 4; ++w) {\n          float a_[4];\n#pragma unroll\n"
              << "          for (int i = 0; i < 4; ++i) a_[i] = " << at(q.qSrc, "rr * EPL + j * VEC + 4 * w + i") << ";\n"
              << "          st_[w] = hf::quant8x4<" << (int)q.lo << ", " << (int)q.hi << ">(a_, " << q.qDiv << ", " << rcp

@@ -288,26 +288,30 @@ __device__ __forceinline__ float lds_chain_sum(const float *rp, float acc) {
 }
 
 // acc + rp[0] + ... + rp[n-1] in that order, for an n that is not the whole
-// chunk: groups of 32 floats, the next group read while one is added.  The
-// floats up to the next multiple of 32 are read too and have to be -0.0 (which
-// no sum notices).  One add per loop turn instead, as this was, waits out the
-// LDS latency every time: softmax 300 x 1001 12.6 -> 6.8 us.
-__device__ __forceinline__ float lds_chain_tail(const float *rp, int n, float acc) {
-  f32x4 a[8], b[8];
-  auto read = [&](f32x4 (&q)[8], int g) {
+// chunk: groups of 4 Q floats, the next group read while one is added.  The
+// floats up to the next multiple of 4 Q are read too and have to be -0.0 (which
+// no sum notices).  One add per loop turn instead waits out the LDS latency
+// every time: softmax 300 x 1001 12.6 -> 6.8 us.  The two groups are 8 Q
+// registers: with 32 rows a block, Q = 8 leaves three waves per SIMD where Q =
+// 4 leaves room for another block (softmax 32768 x 100 16.0 -> 11.3 us); with
+// fewer rows there is no other block, and Q = 8 is up to 5 % the faster
+// (layernorm 2048 x 1001 10.9 and 11.5 us).
+template <int Q> __device__ __forceinline__ float lds_chain_tail(const float *rp, int n, float acc) {
+  f32x4 a[Q], b[Q];
+  auto read = [&](f32x4 (&q)[Q], int g) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const f32x4 *>(rp + 32 * g + 4 * i);
+    for (int i = 0; i < Q; ++i) q[i] = *reinterpret_cast<const f32x4 *>(rp + 4 * (Q * g + i));
   };
-  auto add = [&](const f32x4 (&q)[8]) {
+  auto add = [&](const f32x4 (&q)[Q]) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < Q; ++i) {
       acc = q[i].x + acc;
       acc = q[i].y + acc;
       acc = q[i].z + acc;
       acc = q[i].w + acc;
     }
   };
-  const int ng = (n + 31) / 32;
+  const int ng = (n + 4 * Q - 1) / (4 * Q);
   if (ng > 0) read(a, 0);
   for (int g = 0; g < ng; g += 2) {
     if (g + 1 < ng) read(b, g + 1);
@@ -383,7 +387,7 @@ __device__ __forceinline__ void row_sum_ordered(F val, PF prefetch, const float 
       if (n == CHUNK) {
         acc = lds_chain_sum<CHUNK>(rp, acc);
       } else {
-        acc = lds_chain_tail(rp, n, acc);
+        acc = lds_chain_tail<(RPW == 4 ? 4 : 8)>(rp, n, acc);
       }
     }
     if (k + 1 < NK && wave0) write(k + 1, nxt);

@@ -1262,7 +1262,7 @@ def entries():
     # one kernel for every row count (compiler option dyn=runtime)
     e["rmsnorm_quant_dyn_rt"] = e["rmsnorm_quant_dyn"]
     e["softmax_dyn_rt"] = e["softmax_dyn"]
-    for c in (603, 1000):  # serial-order row schedules by row count, odd and whole chunks
+    for c in (127, 603, 772, 1000):  # serial-order row schedules by row count: odd, 8-byte and whole chunks
         e[f"rmsnorm_quant_w{c}_rt"] = g.with_dynamic_rows(g.rmsnorm_quant(7919, c), 7919)
     e["eltwise_mix_dyn_rt"] = g.with_dynamic_rows(eltwise_mix(67, 1000), 67)
     e["w8a8_dyn_rt"] = g.with_dynamic_rows(g.w8a8_dequant(333, 512, 512), 333)

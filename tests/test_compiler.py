@@ -332,3 +332,28 @@ def test_serial_order_rows_have_one_widest_row(tmp_path):
     # other float sums of wide rows are folded in tree order, unless asked for
     assert emit(hf.groups.safe_softmax(100, 8192), tmp_path)[0] == 0
     assert "does not fit one row group" in emit(hf.groups.safe_softmax(100, 8192), tmp_path, options="ordered_fp_sums=1")[1]
+
+
+def _vec(ir, tmp_path, kernel=""):
+    rc, err, prefix = emit(ir, tmp_path, options="dyn=runtime" if "?" in ir else "")
+    assert rc == 0, err
+    src = open(prefix + ".hip").read().split(f"{kernel}_body(", 1)[1]
+    return int(re.search(r"VEC = (\d+)", src).group(1))
+
+
+def test_access_width_of_serial_order_rows(tmp_path):
+    """Up to 4096 rows a row is read in full-width accesses whatever its
+    length; with more rows narrow ones take the width that divides them (a
+    launch-time row count: one kernel of each kind)."""
+    g = hf.groups
+    for cols, few, many in ((64, 4, 4), (65, 4, 1), (127, 4, 1), (602, 4, 2), (603, 4, 1), (604, 4, 4), (641, 4, 4), (701, 4, 4),
+                            (4095, 4, 4)):
+        assert _vec(g.safe_softmax(4096, cols), tmp_path) == few, cols
+        assert _vec(g.safe_softmax(4097, cols), tmp_path) == many, cols
+    for cols, few, many in ((127, 8, 1), (772, 8, 4), (1280, 8, 8), (1281, 8, 8), (2412, 8, 4), (3332, 8, 8), (4095, 8, 8)):
+        assert _vec(g.rmsnorm_quant(4096, cols), tmp_path) == few, cols
+        assert _vec(g.rmsnorm_quant(4097, cols), tmp_path) == many, cols
+    ir = g.with_dynamic_rows(g.safe_softmax(7919, 127), 7919)
+    assert _vec(ir, tmp_path, "hf_safe_softmax") == 1 and _vec(ir, tmp_path, "hf_safe_softmax_r4096") == 4
+    # (int8 codes at a width below four: the exact pass stores them)
+    assert hf.compile(g.rmsnorm_quant(5000, 127), options="").hsaco

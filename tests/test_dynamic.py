@@ -362,7 +362,7 @@ def test_gpu_runtime_rows_argmax(gpu, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("cols", [603, 1000])
+@pytest.mark.parametrize("cols", [127, 603, 772, 1000])
 def test_gpu_row_schedules(gpu, cols):
     """The serial-order row program's schedules (1 to 32 rows a block), the one
     for each row count through one code object, at the counts where they
