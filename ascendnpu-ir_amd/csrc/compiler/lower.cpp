@@ -4328,7 +4328,42 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
         if (rows && opt.rmsnKernel && matchRmsQuant(A, rq) && !rq.f32x) {
           p = lowerRmsNorm(A, rq, kname);
         } else if (rows && opt.rmsqKernel && matchRmsQuant(A, rq)) {
-          p = lowerRmsQuant(A, rq, kname);
+          // one wave per row, unless the row program is the faster: an f32 row
+          // is twice the bytes of a bf16 one and eight waves fill a CU.  Up to
+          // 2048 rows every row has a wave of its own; from there to 8192 the
+          // row program's blocks (at most 32 rows) are one per CU; past that
+          // they queue, where only rows of 1024 still gain.  us, waves and row
+          // program, before / after each line: of 1024 columns 2048 rows 6.9
+          // and 7.1, 2560 12.8 and 8.4, 8192 18.9 and 12.3, 16384 33.7 and 25.0;
+          // of 2048 columns 2048 rows 9.1 and 11.5, 2560 15.1 and 13.2, 8192 25.3
+          // and 22.9, 9000 28.1 and 36.1; of 4096 columns 4096 rows 24.7 and
+          // 24.6, 8192 38.5 and 116
+          const bool narrow = rq.f32x && A.D[1] < 4096, tall = A.D[1] == 2048;
+          const int64_t R = A.D[0];
+          if (narrow && A.rowsDyn) {
+            auto wave = [&](const std::string &n) { return lowerRmsQuant(A, rq, n); };
+            auto program = [&](const std::string &n, int64_t rows) {
+              RowEmitter e(A, opt);
+              if (rows) e.rowsHint = rows;
+              return e.run(n, "LAST_AXIS_PBR");
+            };
+            const KernelPlan w = tall ? KernelPlan() : wave(kname + "_wave"), q = program(kname + "_r4096", 4096);
+            p = tall ? wave(kname) : program(kname, 0);
+            p.source += w.source + q.source;
+            // (a grid of 256 workgroups for every row count up to 2048)
+            p.alts.push_back({tall ? kname : w.kernelName, 2048, 2048, 256, tall ? p.block[0] : w.block[0]});
+            p.alts.push_back({q.kernelName, 4096, q.rowsB, 1, q.block[0]});
+            if (tall) {
+              const KernelPlan q2 = program(kname + "_r8192", 8192);
+              p.source += q2.source;
+              p.alts.push_back({q2.kernelName, 8192, q2.rowsB, 1, q2.block[0]});
+            }
+          } else if (narrow && R > 2048 && !(tall && R > 8192)) {
+            RowEmitter e(A, opt);
+            p = e.run(kname, "LAST_AXIS_PBR");
+          } else {
+            p = lowerRmsQuant(A, rq, kname);
+          }
         } else if (rows) {
           RowEmitter e(A, opt);
           p = e.run(kname, "LAST_AXIS_PBR");

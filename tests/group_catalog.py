@@ -1272,6 +1272,8 @@ def entries():
     # the norm + quant pattern on an f32 x (as behind a contraction)
     for c in (1024, 2048, 4096):
         e[f"rmsnorm_quant_f32_{c}"] = rmsnorm_quant_f32(256, c)
+    for c in (1024, 2048):
+        e[f"rmsnorm_quant_f32_{c}_rt"] = g.with_dynamic_rows(rmsnorm_quant_f32(7919, c), 7919)
     # every contraction tile through one launch-time row count
     for lay in ("nk", "kn"):
         e[f"tiles_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 1088, b_layout=lay), 7919)

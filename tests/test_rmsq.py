@@ -15,7 +15,7 @@ import pytest
 
 import hfusion_mi355x as hf
 import group_catalog as cat
-from helpers import run_gpu, run_oracle
+from helpers import run_gpu, run_oracle, to_dev
 
 I = hf.inputs
 C = 4096
@@ -175,6 +175,44 @@ def test_rmsq_kernel_takes_f32():
         ir = cat.get(f"rmsnorm_quant_f32_{c}")
         assert "binade-run" in hf.compile(ir).blocks[0]["variant"]
         assert "serial-order" in hf.compile(ir, options="rmsq_kernel=0").blocks[0]["variant"]
+
+
+def test_rmsq_f32_kernel_by_row_count():
+    """An f32 x of 1024 or 2048 columns: a wave per row up to 2048 rows, the
+    row program beyond (of 2048 columns: to 8192 rows), static or launch-time."""
+    wave = lambda b: "binade-run" in b["variant"]
+    for cols, rows, want in ((1024, 2048, True), (1024, 2049, False), (1024, 20000, False), (2048, 2048, True), (2048, 2049, False),
+                             (2048, 8192, False), (2048, 8193, True), (4096, 2049, True), (4096, 8192, True)):
+        assert wave(hf.compile(cat.rmsnorm_quant_f32(rows, cols), options="emit=hip").blocks[0]) == want, (cols, rows)
+        assert wave(hf.compile(hf.groups.rmsnorm_quant(rows, cols), options="emit=hip").blocks[0])
+    for cols, main, alts in ((1024, False, [("_wave", 2048, 256), ("_r4096", 4096, 1)]),
+                             (2048, True, [("", 2048, 256), ("_r4096", 4096, 1), ("_r8192", 8192, 1)])):
+        art = hf.compile(cat.get(f"rmsnorm_quant_f32_{cols}_rt"), options="dyn=runtime;emit=hip")
+        kern = art.blocks[0]["kernel"] if "kernel" in art.blocks[0] else "hf_rmsnorm_quant"
+        got = [ln.split()[1:] for ln in open(art.manifest) if ln.startswith("alt ")]
+        assert wave(art.blocks[0]) == main
+        assert [(a[0], int(a[1]), int(a[3])) for a in got] == [(kern + n, top, c) for n, top, c in alts]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [1024, 2048])
+def test_rmsq_f32_launch_time_rows(gpu, cols):
+    """One code object over both kernels, at the row counts where they change."""
+    base = f32_rows(cols, 2)
+    g = I.uniform_bf16(I.SEED_BASE + 78, (cols,), 0.25, 4.0)
+    name = f"rmsnorm_quant_f32_{cols}_rt"
+    grp = hf.compile(cat.get(name), options="dyn=runtime", require_cached=True).load()
+    rq, rs = run_oracle(f"rmsnorm_quant_f32_{cols}", [base, g, np.zeros((256, cols), np.int8), np.zeros(256, np.float32)])
+    nan = np.isnan(rs)
+    for rows in (1, 9, 256, 2048, 2049, 4096, 4097, 8192, 8193):
+        print(f"[case] {name} rows={rows}", flush=True)
+        at = (np.arange(rows) * 37 + rows) % 256  # the oracle's rows, in another order
+        args = [base[at], g, np.zeros((rows, cols), np.int8), np.zeros(rows, np.float32)]
+        devs = [to_dev(a, p["elem"], gpu) for a, p in zip(args, grp.meta["params"])]
+        q, s = (t.cpu().numpy() for t in grp(*devs))
+        assert np.array_equal(q, rq[at]) and np.array_equal(np.isnan(s), nan[at])
+        ok = ~nan[at]
+        assert np.array_equal(s[ok].view(np.uint32), rs[at][ok].view(np.uint32))
 
 
 @pytest.mark.gpu
