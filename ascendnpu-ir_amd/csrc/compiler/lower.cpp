@@ -2436,22 +2436,33 @@ constexpr int MK_BF16_CODE = 1; // hf::MK_BF16
 
 // The tile of a contraction.  A tile's time is what its CU takes to pull
 // (tm + tn) K bytes through its LDS and multiply them, and 256 CUs work at
-// once: large tiles move fewer bytes, small ones fill the chip.  The times
-// below are measured (us per 4096 bytes of K beyond an empty launch's 2.3 us,
-// W8A8 and bf16 alike at N = 4096): `one` workgroup on a CU, a `second` beside
-// it, each one `more` (0: a CU holds one, the next wait).  Both sides of the
-// lines they draw, W8A8 at N = K = 4096: M = 64: 6.1 us (32x32) against 10.1
-// (64x64); M = 128: 8.5 (64x32) against 10.7 (64x64); M = 200: 10.9 (64x64, two
-// slices a stage) against 11.8 (one); M = 333: 13.5 (64x64, one) against 14.6
-// (128x64, two) and 15.3 (128x64, one), and of a [K, N] B 14.7 (64x128, two)
-// against 16.0 (64x64, one); M = 1024: 22.6 (128x128) against 23.8 (128x64) and
-// 31.6 (256x128); M = 2048: 40.7 (256x128) against 46.1 (128x128 and
-// 256x256); block-scaled fp8, M = 2048: 56.6 (256x256) against 60.9 (128x128).
+// once: large tiles move fewer bytes, small ones fill the chip.  The numbers
+// below are fitted to the times of every tile at M = 16 .. 16384, N = 1024,
+// 4096 and 11008 and K of 1024, 4096 and 8192 bytes (us; W8A8 and bf16 alike,
+// block-scaled ones by format; within 2 to 5 % of the measured times where a
+// tile is near the best).  With n tiles per CU, in rounds of one tile a CU:
+//   time = fixed + queued * (rounds - 1) + K / 4096 bytes * (one for a full
+//          first round, + second for the second, + more for each further one)
+// of which the last, partly filled round takes the share part + (1 - part) *
+// filled^2 (a CU has more of the L2s and the power while others idle; `part1`
+// of the first round, `part` of later ones).  A CU that holds one tile has
+// second = more = one.  More than 18 rows of tiles add up to `tall` of it: fewer
+// of the tiles at work on an XCD share a column of B.
+// Over the measured sizes the picks take 0.2 to 1 % more than the best tile on
+// average, and none over 6 % more than the 256x256 ring.  W8A8, N = K = 4096:
+// M = 64 6.1 us (32x32) against 10.1 (64x64); M = 333 13.5 (64x64) against 15.3
+// (128x64); M = 1024 22.6 (128x128) against 31.6 (256x128); M = 2048 40.7
+// (256x128) against 46.1 (128x128 and 256x256); M = 5000 103 (256x256) against
+// 125 (128x128).  bf16, M = 5000, N = 1024, K = 4096: 60 (256x128) against 65
+// (256x256) and 93 (128x64).
+struct TileTime {
+  double fixed, queued, one, second, more, part1, part, tall;
+};
 struct ContractionTile {
   char kind;           // 's' mmad_skinny, 't' mmad_tile, 'r' the 256x256 ring kernels of hf_mmad.h
   int tm, tn, a, b, s; // 's': a waves; 't': a x b waves per slice of K, s ring stages
-  double one, second, more;
-  int kg = 1;          // 't': slices of K (and groups of a x b waves) per stage
+  int kg;              // 't': slices of K (and groups of a x b waves) per stage
+  TileTime t;
   bool operator==(const ContractionTile &o) const { return kind == o.kind && tm == o.tm && tn == o.tn && kg == o.kg; }
   int threads() const { return kind == 'r' ? 512 : 64 * kg * a * (kind == 's' ? 1 : b); }
   // workgroups of one row of tiles (in eighths: an XCD each)
@@ -2459,43 +2470,67 @@ struct ContractionTile {
     const int64_t t = (N + tn - 1) / tn;
     return kind == 'r' ? t : (t + 7) / 8 * 8;
   }
+  double time(int64_t M, int64_t N, int64_t Kb) const {
+    const double rows = (double)((M + tm - 1) / tm), n = rows * (double)((N + tn - 1) / tn) / 256;
+    const double done = std::max(0.0, std::ceil(n) - 1), filled = n - done; // whole rounds, the last one's share
+    const double last = done == 0 ? t.one : done == 1 ? t.second : t.more, p = done == 0 ? t.part1 : t.part;
+    double work = done == 0 ? 0 : done == 1 ? t.one : t.one + t.second + t.more * (done - 2);
+    work += last * (p + (1 - p) * filled * filled);
+    work *= 1 + t.tall * std::min(1.0, std::max(0.0, (rows - 18) / 16));
+    return t.fixed + t.queued * done + work * (double)Kb / 4096;
+  }
 };
-const ContractionTile kRing256 = {'r', 256, 256, 0, 0, 0, 60, 0, 0};
+const ContractionTile kRing256 = {'r', 256, 256, 0, 0, 0, 1, {}};
 
 ContractionTile pickTile(int64_t M, int64_t N, int64_t Kb, bool bT, int mk) {
   static const std::vector<ContractionTile> nk = {
-      {'s', 16, 16, 8, 0, 0, 2.4, 0, 0},        {'s', 32, 16, 8, 0, 0, 2.8, 0, 0},      {'s', 32, 32, 8, 0, 0, 3.8, 0, 0},
-      {'s', 64, 32, 4, 0, 0, 6.2, 0, 0},        {'t', 64, 64, 2, 2, 3, 7.4, 0, 0, 2},   {'t', 64, 64, 2, 2, 3, 8.8, 5.5, 7.5},
-      {'t', 128, 64, 4, 2, 3, 12, 10, 14},      {'t', 128, 128, 4, 4, 3, 20.5, 0, 0},     {'t', 256, 128, 4, 2, 3, 35, 0, 0},
-      kRing256};
+      {'s', 16, 16, 8, 0, 0, 1, {2.1, 0.69, 1.7, 1.7, 1.7, 0.71, 0.71, 0}},
+      {'s', 32, 16, 8, 0, 0, 1, {2.3, 0.85, 2.1, 2.1, 2.1, 0.72, 0.72, 0}},
+      {'s', 32, 32, 8, 0, 0, 1, {2.7, 1.4, 2.9, 2.9, 2.9, 0.75, 0.75, 0}},
+      {'s', 64, 32, 4, 0, 0, 1, {3.6, 2.1, 4.3, 4.3, 4.3, 0.7, 0.7, 0}},
+      {'t', 64, 64, 2, 2, 3, 2, {3.6, 1.5, 7.7, 7.7, 7.7, 0.87, 0.87, 0.17}},
+      {'t', 64, 64, 2, 2, 3, 1, {3, 0.12, 9.19, 2.4, 6.3, 0.88, 0.62, 0.35}},
+      {'t', 128, 64, 4, 2, 3, 1, {3.71, 0.21, 13.1, 7.47, 11.4, 0.75, 0.64, 0.37}},
+      {'t', 128, 128, 4, 4, 3, 1, {3.95, 2.01, 17.7, 17.7, 17.7, 0.698, 0.698, 0.11}},
+      {'t', 256, 128, 4, 2, 3, 1, {5.99, 3.85, 31.3, 31.3, 31.3, 0.708, 0.708, 0.2}},
+      {'r', 256, 256, 0, 0, 0, 1, {9.2, 9.75, 48.9, 48.9, 48.9, 0.51, 0.51, 0}}};
   // B [K, N]: short pieces of every k-row make the narrow tiles slower
   static const std::vector<ContractionTile> kn = {
-      {'s', 16, 16, 8, 0, 0, 6.9, 0, 0},        {'s', 32, 16, 8, 0, 0, 7.4, 0, 0},      {'s', 32, 32, 8, 0, 0, 8.6, 0, 0},
-      {'t', 32, 64, 1, 2, 4, 9, 5, 6},          {'t', 64, 64, 2, 2, 3, 9.6, 0, 0, 2},   {'t', 64, 64, 2, 2, 3, 10.9, 6.5, 8},
-      {'t', 64, 128, 2, 4, 3, 12.2, 0, 0, 2},   {'t', 128, 64, 4, 2, 3, 13, 13, 14.5},  {'t', 128, 128, 4, 4, 3, 19.5, 0, 0},
-      {'t', 256, 128, 4, 2, 3, 36.5, 0, 0},     kRing256};
-  // block-scaled (the scaled instruction takes wider wave tiles)
+      {'s', 16, 16, 8, 0, 0, 1, {2, 0.24, 4.7, 4.7, 4.7, 0.55, 0.55, 0.2}},
+      {'s', 32, 16, 8, 0, 0, 1, {2.1, 0.41, 5.2, 5.2, 5.2, 0.55, 0.55, 0.2}},
+      {'s', 32, 32, 8, 0, 0, 1, {2.4, 0.45, 6.6, 6.6, 6.6, 0.75, 0.75, 0}},
+      {'t', 32, 64, 1, 2, 4, 1, {2.8, 0.33, 8.8, 0.82, 4.1, 0.89, 0.6, 0.1}},
+      {'t', 64, 64, 2, 2, 3, 2, {3.3, 1.3, 8.7, 8.7, 8.7, 0.84, 0.84, 0.14}},
+      {'t', 64, 64, 2, 2, 3, 1, {2.9, 0.19, 10, 3, 6.6, 0.87, 0.63, 0.35}},
+      {'t', 64, 128, 2, 4, 3, 2, {4.7, 2.5, 11.2, 11.2, 11.2, 0.84, 0.84, 0.055}},
+      {'t', 128, 64, 4, 2, 3, 1, {3.1, 0.28, 12.8, 8.2, 12, 0.83, 0.7, 0.31}},
+      {'t', 128, 128, 4, 4, 3, 1, {4.4, 2.2, 18.3, 18.3, 18.3, 0.73, 0.73, 0.069}},
+      {'t', 256, 128, 4, 2, 3, 1, {6, 4.2, 32, 32, 32, 0.76, 0.76, 0.2}},
+      {'r', 256, 256, 0, 0, 0, 1, {9.3, 9.2, 50, 50, 50, 0.53, 0.53, 0}}};
+  // block-scaled (the scaled instruction takes wider wave tiles; a CU holds
+  // two or three of the tiles below 128x128)
   static const std::vector<ContractionTile> fp8 = {
-      {'t', 32, 64, 1, 2, 4, 8, 0, 0}, {'t', 64, 64, 2, 2, 3, 12, 0, 0}, {'t', 64, 128, 2, 2, 3, 15.3, 0, 0},
-      {'t', 128, 128, 4, 2, 3, 28.5, 0, 0}, {'r', 256, 256, 0, 0, 0, 75, 0, 0}};
+      {'t', 32, 64, 1, 2, 4, 1, {2.3, 0, 10.8, 6.4, 7.8, 0.82, 0.65, 0}},
+      {'t', 64, 64, 2, 2, 3, 1, {2.3, 0, 13.7, 7.9, 9.8, 0.81, 0.9, 0.076}},
+      {'t', 64, 128, 2, 2, 3, 1, {3, 0, 17.4, 13.5, 14.4, 0.85, 0.71, 0.09}},
+      {'t', 128, 128, 4, 2, 3, 1, {3.4, 1.7, 28.6, 28.6, 28.6, 0.83, 0.83, 0.081}},
+      {'r', 256, 256, 0, 0, 0, 1, {11, 10.2, 58.1, 58.1, 58.1, 0.7, 0.7, 0}}};
   static const std::vector<ContractionTile> fp4 = {
-      {'t', 32, 64, 1, 2, 4, 9, 0, 0}, {'t', 64, 64, 2, 2, 3, 13, 0, 0}, {'t', 64, 128, 2, 4, 3, 19, 0, 0},
-      {'t', 128, 128, 4, 2, 3, 30, 0, 0}, {'r', 256, 256, 0, 0, 0, 102, 0, 0}};
+      {'t', 32, 64, 1, 2, 4, 1, {2.2, 0, 11.2, 8, 9.8, 0.87, 0.62, 0}},
+      {'t', 64, 64, 2, 2, 3, 1, {2.6, 0, 14, 8.7, 10.9, 0.8, 0.8, 0.11}},
+      {'t', 64, 128, 2, 4, 3, 1, {2.9, 0, 20.2, 15.6, 16.7, 0.84, 0.83, 0.12}},
+      {'t', 128, 128, 4, 2, 3, 1, {4.1, 2.1, 28.1, 28.1, 28.1, 0.81, 0.81, 0.086}},
+      {'r', 256, 256, 0, 0, 0, 1, {10.4, 10.2, 71.9, 71.9, 71.9, 0.66, 0.66, 0}}};
   const std::vector<ContractionTile> &cand = mk == 7 ? fp4 : mk >= 3 ? fp8 : bT ? nk : kn;
   const ContractionTile *best = nullptr;
-  double bestCost = 0;
+  double bestTime = 0;
   for (const ContractionTile &t : cand) {
     // (the 256x256 ring of 64-byte slices took 650 us at M = 3000, N = 4096,
     // K = 4032, where the 256x128 tiles take 76)
     if (t.kind == 'r' && Kb % 128 != 0) continue;
     if (t.kg > 1 && Kb < 1024) continue; // (the groups' sums cost more than they save)
-    const double n = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn) / 256;
-    double cost = n <= 1 ? t.one : !t.second ? t.one * std::ceil(n) : n <= 2 ? t.one + t.second * (n - 1) : t.one + t.second + t.more * (n - 2);
-    // the ring kernels leave the other CUs' power and L2 to the busy ones:
-    // with an eighth or a half of the CUs busy a tile takes 0.67 or 0.75 of
-    // its time with all of them
-    if (t.kind == 'r' && n < 1) cost *= 0.67 + 0.33 * n * n;
-    if (!best || cost < bestCost) { best = &t; bestCost = cost; }
+    const double us = t.time(M, N, Kb);
+    if (!best || us < bestTime) { best = &t; bestTime = us; }
   }
   return *best;
 }
@@ -2774,33 +2809,49 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
     if (mx) k << ", (const uint8_t*)p" << sa->argIdx << ", (const uint8_t*)p" << sb->argIdx;
     k << ", (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
   };
+  // the 256x256 ring on operands as they lie (128-byte slices)
+  auto ringCall = [&]() {
+    if (mx)
+      k << "  hf::mmad_mx<" << mk << ", " << kname << "_epi>((const uint8_t*)p" << a->argIdx << ", (const uint8_t*)p" << b->argIdx
+        << ", (const uint8_t*)p" << sa->argIdx << ", (const uint8_t*)p" << sb->argIdx;
+    else
+      k << "  hf::mmad<" << mk << ", " << kname << "_epi, false, " << (bT ? "true, 3" : "false, 4") << ">((const " << et << "*)p"
+        << a->argIdx << ", (const " << et << "*)p" << b->argIdx;
+    k << ", (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
+  };
   // a runtime row count: the tile that each count would be given, up to the
-  // first that takes the main kernel's 256x256 ring
+  // last that differs from the main kernel's
   if (A.rowsDyn && tiles) {
-    std::vector<ContractionTile> emitted;
+    std::vector<ContractionTile> seq, emitted;
+    std::vector<int64_t> top;
     for (int64_t m = 16; m <= 16384; m += m < 64 ? 16 : 64) {
       const ContractionTile t = pickTile(m, N, K * esz, bT, mk);
-      if (t.kind == 'r') break;
-      const std::string nm = kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn) + (t.kg > 1 ? "k" + std::to_string(t.kg) : "");
-      if (!p.alts.empty() && p.alts.back().name == nm) { p.alts.back().maxRows = m; continue; }
-      if (std::find(emitted.begin(), emitted.end(), t) == emitted.end()) {
+      if (!seq.empty() && seq.back() == t) { top.back() = m; continue; }
+      seq.push_back(t);
+      top.push_back(m);
+    }
+    if (seq.back() == tile) seq.pop_back();
+    for (size_t i = 0; i < seq.size(); ++i) {
+      const ContractionTile &t = seq[i];
+      const bool main = ring && t == tile;
+      const std::string nm = main ? kname : kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn) + (t.kg > 1 ? "k" + std::to_string(t.kg) : "");
+      if (!main && std::find(emitted.begin(), emitted.end(), t) == emitted.end()) {
         emitted.push_back(t);
         kernelHead(nm, t.threads());
-        tileCall(t);
+        if (t.kind == 'r') ringCall();
+        else tileCall(t);
       }
-      p.alts.push_back({nm, m, t.tm, t.blocksPerRow(N), (unsigned)t.threads()});
+      p.alts.push_back({nm, top[i], t.tm, t.blocksPerRow(N), (unsigned)t.threads()});
     }
   }
   kernelHead(kname, threads);
   if (!ring)
     tileCall(tile);
+  else if (tiles)
+    ringCall();
   else if (mxExact)
     k << "  hf::mmad<" << MK_BF16_CODE << ", " << kname << "_epi, false, false, 4>((const uint16_t*)ws, (const uint16_t*)((char*)ws + "
       << wsXA << "), (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
-  else if (mx)
-    k << "  hf::mmad_mx<" << mk << ", " << kname << "_epi>((const uint8_t*)p" << a->argIdx << ", (const uint8_t*)p" << b->argIdx
-      << ", (const uint8_t*)p" << sa->argIdx << ", (const uint8_t*)p" << sb->argIdx << ", (" << mtype(oe) << "*)"
-      << resultPtr(A, 0) << ", " << Mx << ", " << N << "ll, " << K << "ll, P);\n}\n";
   else
     k << "  hf::mmad<" << mk << ", " << kname << "_epi, " << (mT ? "true" : "false") << ", " << (kT ? "true" : "false") << ", "
       << dma << ">(" << aPtr << ", " << bPtr << ", (" << mtype(oe) << "*)" << resultPtr(A, 0) << ", " << Mx << ", " << N

@@ -37,6 +37,23 @@ def test_alternatives_by_row_count():
             assert blk["grid"][0] == -(-int(top) // tm) * int(rc)
 
 
+def test_tile_where_large_ones_queue():
+    """Sizes a little past whole rounds of 256x256 tiles, and few wide columns:
+    the 256x256 ring, or the largest tile that fills the chip."""
+    g = hf.groups
+    ring = "LDS DMA ring (128-byte slices, 2 waves/SIMD"
+    for ir, want in [(g.w8a8_dequant(5000, 4096, 4096), ring), (g.w8a8_dequant(5000, 4096, 4096, b_layout="kn"), ring),
+                     (g.bf16_mmad(5000, 4096, 4096), ring), (g.bf16_mmad(3000, 11008, 4096, b_layout="kn"), ring),
+                     (g.w8a8_dequant(1536, 14336, 4096), ring), (g.matmul_mx(5000, 4096, 4096), "mfma_scale"),
+                     (g.bf16_mmad(5000, 1024, 4096), "256x128 tiles"), (g.w8a8_dequant(5000, 1024, 4096, b_layout="kn"), "256x128 tiles"),
+                     (g.w8a8_dequant(2048, 4096, 4096), "256x128 tiles"), (g.w8a8_dequant(1024, 4096, 4096), "128x128 tiles")]:
+        b = hf.compile(ir, options="emit=hip").blocks[0]
+        assert want in b["variant"], b["variant"]
+    for fmt in ("e4m3", "e2m1"):
+        b = hf.compile(g.matmul_mx(5000, 4096, 4096, fa=fmt, fb=fmt, via="format"), options="emit=hip").blocks[0]
+        assert b["grid"][0] == 20 * 16 and b["block"][0] == 512
+
+
 def _mm(rng, m, k, layout):
     a = rng.integers(-127, 128, (m, k), dtype=np.int8)
     b = rng.integers(-127, 128, (N, k) if layout == "nk" else (k, N), dtype=np.int8)
