@@ -1228,6 +1228,14 @@ def entries():
     e["hivm_mm_i8_at_kn"] = g.hivm_matmul(256, 208, 384, elem="i8", out="bf16", descale="f32",
                                           descale_mode="DescalePerTensor", a_t=True)
     e["hivm_mm_bf16_at_bt"] = g.hivm_matmul(200, 136, 128, elem="bf16", out="f32", a_t=True, b_t=True)
+    # K of an odd number of 64-byte pieces: A [K, M] (and B [K, N]) copied
+    # K-contiguous, then the 64-byte ring, over several ragged 256x256 tiles
+    e["hivm_mm_i8_at_p64"] = g.hivm_matmul(528, 400, 320, elem="i8", out="bf16", descale="f32", descale_mode="DescalePerChannel",
+                                           a_t=True, b_t=True)
+    e["hivm_mm_i8_at_kn_p64"] = g.hivm_matmul(272, 528, 192, elem="i8", out="bf16", descale="f32",
+                                              descale_mode="DescalePerTensor", a_t=True)
+    e["hivm_mm_bf16_at_p64"] = g.hivm_matmul(264, 296, 96, elem="bf16", out="f32", a_t=True)
+    e["hivm_mm_bf16_at_bt_p64"] = g.hivm_matmul(520, 268, 160, elem="bf16", out="f32", a_t=True, b_t=True)
     e["hivm_mm_f16_at_bt"] = g.hivm_matmul(152, 264, 192, elem="f16", out="f16", a_t=True, b_t=True)
     e["mm_i8_ragged"] = g.mm_i8(300, 200, 192)
     e["bf16_mmad_256"] = g.bf16_mmad(256, 256, 256)
@@ -1280,6 +1288,16 @@ def entries():
         e[f"tiles_bf16_{lay}_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 224, b_layout=lay), 7919)
         # ... and the ones of two slices a stage, with 8.5 slices
         e[f"tiles_bf16_{lay}_k544_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 544, b_layout=lay), 7919)
+    for lay in ("nk", "kn"):  # K enough for the tiles of two slices a stage (16.5 slices)
+        e[f"tiles_w8a8_{lay}_k2112_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 1040, 2112, b_layout=lay), 7919)
+        e[f"tiles_bf16_{lay}_k1056_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 1040, 1056, b_layout=lay), 7919)
+        # the ring as the main kernel and between smaller tiles (5 slices, ragged columns)
+        e[f"ring_w8a8_{lay}_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 4016, 640, b_layout=lay), 7919)
+    e["ring_bf16_kn_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 4016, 320, b_layout="kn"), 7919)
+    e["ring_mx_e4m3_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 4016, 640, via="format"), 7919)
+    e["ring_mx_e2m1_rt"] = g.with_dynamic_rows(g.matmul_mx(7919, 4016, 1280, fa="e2m1", fb="e2m1", via="format"), 7919)
+    e["tiles_w8a8_kn_n2064_rt"] = g.with_dynamic_rows(g.w8a8_dequant(7919, 2064, 4160, b_layout="kn"), 7919)
+    e["tiles_bf16_kn_n2064_rt"] = g.with_dynamic_rows(g.bf16_mmad(7919, 2064, 2080, b_layout="kn"), 7919)
     # the 256x256 ring with one to three slices of K, ragged tiles
     e["ring_w8a8_nk_k128"] = g.w8a8_dequant(4000, 4016, 128)
     e["ring_w8a8_kn_k256"] = g.w8a8_dequant(4000, 4016, 256, b_layout="kn")

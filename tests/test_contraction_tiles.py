@@ -1,9 +1,10 @@
 """GPU: every tile of the contraction kernels.
 
 One code object per group takes the row count M at launch and runs the tile
-the lowering chooses for it (16x16 ... 256x128, then the 256x256 ring); N = 1040
-leaves every tile a ragged last column tile, K ends in half a 128-byte slice,
-and the row counts sit on and beside the tiles' edges.  Whole-number sums are
+the lowering chooses for it (16x16 ... 256x128); N = 1040 leaves every tile a
+ragged last column tile, K ends in half a 128-byte slice, and the row counts
+sit on and beside the tiles' edges.  Groups of N = 4016 and whole slices of K
+reach the 256x256 ring, which takes no half slice.  Whole-number sums are
 exact; 16-bit floats are held to the f32 summation bound K 2^-24 sum|ab| plus
 half an ulp of the output; block-scaled results to the matrix core's bars.
 """
@@ -52,6 +53,125 @@ def test_tile_where_large_ones_queue():
     for fmt in ("e4m3", "e2m1"):
         b = hf.compile(g.matmul_mx(5000, 4096, 4096, fa=fmt, fb=fmt, via="format"), options="emit=hip").blocks[0]
         assert b["grid"][0] == 20 * 16 and b["block"][0] == 512
+
+
+TILES = {"nk": {"16x16", "32x16", "32x32", "64x32", "64x64k2", "64x64", "128x64", "128x128", "256x128"},
+         "kn": {"16x16", "32x16", "32x32", "32x64", "64x64k2", "64x64", "64x128k2", "128x64", "128x128", "256x128"},
+         "mx_e4m3": {"32x64", "64x64", "64x128", "128x128"}, "mx_e2m1": {"32x64", "64x64", "64x128", "128x128"}}
+# groups that between them run every tile of a family: (name, N, K)
+TILE_GROUPS = {("nk", "w8a8"): [("tiles_w8a8_nk_k2112_rt", 1040, 2112)], ("nk", "bf16"): [("tiles_bf16_nk_k1056_rt", 1040, 1056)],
+               ("kn", "w8a8"): [("tiles_w8a8_kn_k2112_rt", 1040, 2112), ("tiles_w8a8_kn_rt", 1040, 1088), ("tiles_w8a8_kn_n2064_rt", 2064, 4160)],
+               ("kn", "bf16"): [("tiles_bf16_kn_k1056_rt", 1040, 1056), ("tiles_bf16_kn_k544_rt", 1040, 544), ("tiles_bf16_kn_n2064_rt", 2064, 2080)],
+               ("mx_e4m3", ""): [("tiles_mx_e4m3_rt", 1040, 640)], ("mx_e2m1", ""): [("tiles_mx_e2m1_rt", 1040, 1280)]}
+MOST_ROWS = 6000
+RING_GROUPS = ["ring_w8a8_nk_rt", "ring_w8a8_kn_rt", "ring_bf16_kn_rt", "ring_mx_e4m3_rt", "ring_mx_e2m1_rt"]
+
+
+def _alts(name, **kw):
+    """(kernel, largest row count, rows a tile) of each alternative, ascending."""
+    art = hf.compile(cat.get(name), options="dyn=runtime", **kw)
+    rows = [ln.split()[1:] for ln in open(art.manifest) if ln.startswith("alt ")]
+    return [(r[0], int(r[1]), int(r[2])) for r in rows]
+
+
+def _rows_of_tiles(name, **kw):
+    """{tile: the first and the last row count of its first range}."""
+    out, low = {}, 0
+    for kern, top, _ in _alts(name, **kw):
+        out.setdefault(kern.rsplit("_", 1)[1], (low + 1, top))
+        low = top
+    return out
+
+
+def _ring_rows(name, **kw):
+    """Row counts that run the main kernel (the ring): the first and the last
+    of its first range as an alternative, and one past every alternative."""
+    alts, low, rows = _alts(name, **kw), 0, []
+    for kern, top, tm in alts:
+        if tm == 256 and "_256x" not in kern and not rows:
+            rows = [low + 1, top]
+        low = top
+    return rows + [low + 1, low + 300]
+
+
+@pytest.mark.parametrize("family", list(TILE_GROUPS))
+def test_every_tile_is_picked(family):
+    """The groups run every tile that the lowering can pick, each within the
+    row counts that the GPU test takes."""
+    run = {t for name, _, _ in TILE_GROUPS[family] for t, ends in _rows_of_tiles(name).items() if ends[0] <= MOST_ROWS}
+    assert run - {"256x256"} == TILES[family[0]]
+
+
+def test_ring_rows_run_the_ring():
+    for name in RING_GROUPS:
+        b = hf.compile(cat.get(name), options="dyn=runtime").blocks[0]
+        assert b["rows_dyn"][1] == 256 and b["rows_dyn"][2] == -(-4016 // 256) and b["block"][0] == 512, name
+        assert len(_ring_rows(name)) >= 2 and max(_ring_rows(name)) < 20000
+
+
+def _whole(name, m, n, k, gpu, seed):
+    """A group over whole numbers whose sums are exact in any order, checked
+    against the 64-bit product."""
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    ints = lambda lo, hi, *sh: torch.randint(lo, hi + 1, sh, device=gpu, generator=gen)
+    kind = "mx" if "_mx_" in name else "bf16" if "_bf16_" in name else "w8a8"
+    dg = hf.DynamicGroup(cat.get(name), require_cached=True, runtime=True)
+    if kind == "mx":
+        # e4m3 0 .. 7 and e2m1 0 .. 6 by magnitude, scales 1/2, 1 and 2 per 32 k:
+        # multiples of 1/4 with |sum| <= 196 K < 2^22 of them
+        fp4 = "e2m1" in name
+        code = torch.tensor([0x0, 0x2, 0x4, 0x5, 0x6, 0x7] if fp4 else [0x00, 0x38, 0x40, 0x44, 0x48, 0x4A, 0x4C, 0x4E], device=gpu)
+        val = torch.tensor([0, 1, 2, 3, 4, 6] if fp4 else [0, 1, 2, 3, 4, 5, 6, 7], dtype=torch.float64, device=gpu)
+        def operand(*sh):
+            i, neg = ints(0, len(code) - 1, *sh), ints(0, 1, *sh)
+            return code[i] + neg * (8 if fp4 else 128), val[i] * (1 - 2 * neg)
+        (ca, va), (cb, vb) = operand(m, k), operand(k, n)
+        sa, sb = ints(126, 128, m, k // 32), ints(126, 128, n, k // 32)
+        ref = (va * torch.exp2(sa.double() - 127).repeat_interleave(32, 1)) @ (vb * torch.exp2(sb.double() - 127).repeat_interleave(32, 1).t())
+        if fp4:
+            ca, cb = ca[:, 0::2] | ca[:, 1::2] << 4, cb[0::2] | cb[1::2] << 4
+        by = lambda t: t.to(torch.uint8).view(torch.int8).contiguous()
+        return dg(by(ca), by(cb), by(sa), by(sb)).double(), ref
+    lim = 127 if kind == "w8a8" else 3
+    a, b = ints(-lim, lim, m, k), ints(-lim, lim, *((n, k) if "_nk_" in name else (k, n)))
+    c = a.double() @ (b.double().t() if "_nk_" in name else b.double())
+    if kind == "bf16":
+        out = dg(a.bfloat16(), b.bfloat16(), torch.empty(m, n, dtype=torch.bfloat16, device=gpu))
+        return out, c.bfloat16()
+    # (scales are powers of two: one rounding, to bf16; |c| <= 127^2 K rounds to f32 first)
+    st, sc = torch.exp2(ints(-6, 0, m).float()), torch.exp2(ints(-6, 0, n).float())
+    out = dg(a.to(torch.int8), b.to(torch.int8), st, sc, torch.empty(m, n, dtype=torch.bfloat16, device=gpu))
+    return out, ((c.float() * st[:, None]) * sc[None, :]).bfloat16()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,n,k", [g for v in TILE_GROUPS.values() for g in v])
+def test_gpu_every_tile(gpu, name, n, k):
+    """Every tile of a group at the ends of its first range of row counts,
+    ragged in N, K and M."""
+    import torch
+    for tile, ends in _rows_of_tiles(name, require_cached=True).items():
+        for m in ends:
+            if m > MOST_ROWS:
+                continue
+            print(f"[case] {name} {tile} M={m}", flush=True)
+            out, ref = _whole(name, m, n, k, gpu, 91 + m)
+            assert torch.equal(out, ref), (tile, m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", RING_GROUPS)
+def test_gpu_ring_launch_time_rows(gpu, name):
+    """The 256x256 ring with a launch-time row count, where the alternatives
+    hand over to it and past them."""
+    import torch
+    k = {"w8a8": 640, "bf16": 320, "e4m3": 640, "e2m1": 1280}[name.split("_")[2 if "_mx_" in name else 1]]
+    for m in _ring_rows(name, require_cached=True):
+        print(f"[case] {name} M={m}", flush=True)
+        out, ref = _whole(name, m, 4016, k, gpu, 92 + m)
+        assert torch.equal(out, ref), m
+        del out, ref
 
 
 def _mm(rng, m, k, layout):

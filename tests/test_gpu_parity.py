@@ -217,6 +217,30 @@ def _hivm_inputs(name):
     raise KeyError(name)
 
 
+@pytest.mark.parametrize("name,m,n,k,bt", [("hivm_mm_i8_at_p64", 528, 400, 320, True), ("hivm_mm_i8_at_kn_p64", 272, 528, 192, False),
+                                           ("hivm_mm_bf16_at_p64", 264, 296, 96, False), ("hivm_mm_bf16_at_bt_p64", 520, 268, 160, True)])
+def test_hivm_matmul_copied_operands(gpu, name, m, n, k, bt):
+    """A [K, M] with K an odd number of 64-byte pieces: the operands copied
+    K-contiguous by the transpose kernel, then the 64-byte ring."""
+    note(name)
+    v = hf.compile(cat.get(name), require_cached=True).blocks[0]["variant"]
+    assert "re-laid K-contiguous by a transpose kernel" in v and v.endswith(", LDS DMA ring"), v
+    s, i8 = I.SEED_BASE + 49, "_i8_" in name
+    mk = I.int8_uniform if i8 else I.normal_bf16
+    args = [mk(s, (k, m)), mk(s + 1, (n, k) if bt else (k, n))]
+    if i8:
+        args.append(I.uniform_f32(s + 2, (n,) if bt else (1,), 0.001, 0.02))
+    args.append(np.zeros((m, n), np.uint16 if i8 else np.float32))
+    out, = run_gpu(name, args, gpu)
+    ref, = run_oracle(name, args)
+    if i8:
+        assert np.array_equal(out, ref)
+    else:  # f32 sums in another order: K 2^-24 of the products' magnitude sum, each side
+        fa, fb = (np.abs(I.bf16_bits_to_f32(x)).astype(np.float64) for x in args[:2])
+        mag = fa.T @ (fb.T if bt else fb)
+        assert np.all(np.abs(out.astype(np.float64) - ref) <= 2 * k * 2.0 ** -24 * mag)
+
+
 @pytest.mark.parametrize("name", ["hivm_mm_f16_null", "hivm_mm_f16_bias_pc", "hivm_mm_f16_bias_pt_t", "hivm_mm_i8_pc",
                                   "hivm_mm_i8_pt_i8out", "hivm_mm_bf16_at", "hivm_mm_i8_at", "hivm_mm_i8_at_kn",
                                   "hivm_mm_bf16_at_bt", "hivm_mm_f16_at_bt"])
