@@ -231,3 +231,26 @@ def test_rmsq_f32_bit_exact(gpu, cols, seed):
         f"scales differ in rows {np.nonzero(s.view(np.uint32) != rs.view(np.uint32))[0][:16]}"
     bad = np.nonzero((q != rq).any(axis=1))[0]
     assert bad.size == 0, f"codes differ in rows {bad[:16]}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [1024, 2048, 4096])
+def test_rmsq_f32_views_at_any_element(gpu, cols):
+    """x, gamma, codes and scales at element offsets of 1 to 3 behind an
+    allocation: the bits of the aligned call."""
+    import torch
+    name = f"rmsnorm_quant_f32_{cols}"
+    print(f"[case] {name} views", flush=True)
+    grp = hf.compile(cat.get(name), require_cached=True).load()
+    x = to_dev(f32_rows(cols, 3), "f32", gpu)
+    g = to_dev(I.uniform_bf16(I.SEED_BASE + 77, (cols,), 0.25, 4.0), "bf16", gpu)
+    new = lambda: (torch.zeros(256, cols, dtype=torch.int8, device=gpu), torch.zeros(256, device=gpu))
+    def moved(t, off):
+        buf = torch.full((t.numel() + 8,), 85, dtype=t.dtype, device=gpu)
+        v = buf[off:off + t.numel()].view(t.shape)
+        v.copy_(t)
+        return v
+    q, s = grp(x, g, *new())
+    for off in (1, 2, 3):
+        q2, s2 = grp(moved(x, off), moved(g, off), *(moved(t, off) for t in new()))
+        assert torch.equal(q2, q) and torch.equal(s2.view(torch.int32), s.view(torch.int32)), off
