@@ -40,13 +40,13 @@ __device__ __forceinline__ uint64_t rec_pack(float m, uint32_t j, bool has_nan) 
 }
 // Reads a record whose writer has counted itself in, and clears it.  The
 // word is on its way if not there yet; the wait is bounded all the same, so
-// that launches which overlap on one workspace against its rule give wrong
-// values (an empty record) and not a hang.
+// that launches which overlap on one workspace against its rule cannot hang.
+// 0: it did not arrive.
 __device__ __forceinline__ uint64_t rec_take(uint64_t *slot) {
   uint64_t w = 0;
   for (int t = 0; t < (1 << 16) && !(w >> 63); ++t) w = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __hip_atomic_store(slot, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return w >> 63 ? w : rec_pack(0.0f, ARG_EMPTY, false);
+  return w >> 63 ? w : 0;
 }
 
 template <int KIND> __device__ __forceinline__ bool arg_better(float a, float b) { return KIND == 0 ? (a > b) : (a < b); }
@@ -274,10 +274,12 @@ __device__ void arg_item(const float *__restrict__ x, int64_t R, int64_t C, int6
   // first that holds a NaN do not count
   uint64_t rec[8];
   int64_t firstNan = INT64_MAX;
+  bool lost = false;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int64_t t = lane + 64 * k;
     rec[k] = 64 * k < SEG && t < SEG ? rec_take(&recs[row * SEG + t]) : rec_pack(0.0f, ARG_EMPTY, false);
+    lost |= rec[k] == 0;
     if (firstNan == INT64_MAX && (rec[k] >> 62 & 1)) firstNan = t;
   }
 #pragma unroll
@@ -299,6 +301,7 @@ __device__ void arg_item(const float *__restrict__ x, int64_t R, int64_t C, int6
     const int64_t j2 = __shfl_xor(jx, sh, 64);
     arg_combine<KIND>(m, jx, m2, j2);
   }
+  const bool anyLost = __ballot(lost) != 0;
   if (lane != 0) return;
   float V = init_v;
   int64_t I = (int64_t)init_i;
@@ -308,6 +311,10 @@ __device__ void arg_item(const float *__restrict__ x, int64_t R, int64_t C, int6
       V = arg_fold<KIND>(m, V);
     }
     if (firstNan != INT64_MAX) V = __builtin_nanf("");
+  }
+  if (anyLost) { // the row says so: no index of its own, no number
+    V = __builtin_nanf("");
+    I = -1;
   }
   if (out_v) out_v[row] = V;
   if (out_i) out_i[row] = (IdxT)I;

@@ -282,3 +282,33 @@ def test_plain_call_checks_and_stream(gpu):
     assert not done.query()
     side.synchronize()
     assert float(o.min()) == 2.0
+
+
+def test_argmax_record_that_never_arrives(gpu):
+    """One workgroup of a split-row argmax by hand, its row's counter set so
+    that it takes itself for the last: the bounded wait for the other segments'
+    records ends, and the row says that it has no result (NaN, -1)."""
+    import torch
+    note("argmax_16 one segment alone")
+    art = hf.compile(cat.get("argmax_16"), require_cached=True)
+    blk = art.blocks[0]
+    segs = blk["grid"][0] // 16
+    assert segs > 1
+    lib = native.hfr()
+    mod, kern = ctypes.c_void_p(), ctypes.c_void_p()
+    native.check(lib.hfr_module_load(art.hsaco.encode(), ctypes.byref(mod)))
+    native.check(lib.hfr_kernel_get(mod, b"hf_argmax", ctypes.byref(kern)))
+    x = torch.randn(16, 152064, device=gpu)
+    v, i = torch.zeros(16, device=gpu), torch.zeros(16, dtype=torch.int32, device=gpu)
+    ws = torch.zeros(blk["workspace"] // 4, dtype=torch.int32, device=gpu)
+    ws[16 * segs * 2] = segs - 1  # (16 segs records of 8 bytes, then the rows' counters)
+    slot = {"param:0": x.data_ptr(), "param:1": v.data_ptr(), "param:2": i.data_ptr(), "ws": ws.data_ptr()}
+    args = (ctypes.c_uint64 * len(blk["kargs"]))(*[slot[k] for k in blk["kargs"]])
+    cfg = native.LaunchCfg((ctypes.c_uint * 3)(1, 1, 1), (ctypes.c_uint * 3)(*blk["block"]), 0)
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    torch.cuda.synchronize()
+    native.check(lib.hfr_launch(kern, ctypes.byref(cfg), args, len(args), stream))
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(v[0])) and int(i[0]) == -1
+    assert not v[1:].any() and not i[1:].any() and not ws.any()
+    native.check(lib.hfr_module_unload(mod))
