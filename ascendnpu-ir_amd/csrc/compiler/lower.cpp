@@ -2432,6 +2432,10 @@ void hivmMatmulEpilogue(const Op *mm, bool intAcc, std::ostringstream &epi, std:
   else unsupported(mm, "matmul output type");
 }
 
+// The kernel of a group for some of its row counts: no function's own kernel
+// ("hf_" and its name) is called so, whatever the function's name.
+std::string altName(const std::string &kname, const std::string &what) { return "hfa_" + kname.substr(3) + "_" + what; }
+
 constexpr int MK_BF16_CODE = 1; // hf::MK_BF16
 
 // The tile of a contraction.  A tile's time is what its CU takes to pull
@@ -2834,7 +2838,7 @@ KernelPlan lowerMatmul(Analysis &A, const std::string &kname, const LowerOptions
     for (size_t i = 0; i < seq.size(); ++i) {
       const ContractionTile &t = seq[i];
       const bool main = ring && t == tile;
-      const std::string nm = main ? kname : kname + "_" + std::to_string(t.tm) + "x" + std::to_string(t.tn) + (t.kg > 1 ? "k" + std::to_string(t.kg) : "");
+      const std::string nm = main ? kname : altName(kname, std::to_string(t.tm) + "x" + std::to_string(t.tn) + (t.kg > 1 ? "k" + std::to_string(t.kg) : ""));
       if (!main && std::find(emitted.begin(), emitted.end(), t) == emitted.end()) {
         emitted.push_back(t);
         kernelHead(nm, t.threads());
@@ -4398,14 +4402,14 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
               if (rows) e.rowsHint = rows;
               return e.run(n, "LAST_AXIS_PBR");
             };
-            const KernelPlan w = tall ? KernelPlan() : wave(kname + "_wave"), q = program(kname + "_r4096", 4096);
+            const KernelPlan w = tall ? KernelPlan() : wave(altName(kname, "wave")), q = program(altName(kname, "r4096"), 4096);
             p = tall ? wave(kname) : program(kname, 0);
             p.source += w.source + q.source;
             // (a grid of 256 workgroups for every row count up to 2048)
             p.alts.push_back({tall ? kname : w.kernelName, 2048, 2048, 256, tall ? p.block[0] : w.block[0]});
             p.alts.push_back({q.kernelName, 4096, q.rowsB, 1, q.block[0]});
             if (tall) {
-              const KernelPlan q2 = program(kname + "_r8192", 8192);
+              const KernelPlan q2 = program(altName(kname, "r8192"), 8192);
               p.source += q2.source;
               p.alts.push_back({q2.kernelName, 8192, q2.rowsB, 1, q2.block[0]});
             }
@@ -4423,7 +4427,7 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
             for (int64_t rows : {256, 512, 1024, 2048, 4096}) {
               RowEmitter few(A, opt);
               few.rowsHint = rows;
-              const KernelPlan q = few.run(kname + "_r" + std::to_string(rows), "LAST_AXIS_PBR");
+              const KernelPlan q = few.run(altName(kname, "r" + std::to_string(rows)), "LAST_AXIS_PBR");
               p.source += q.source;
               p.alts.push_back({q.kernelName, rows, q.rowsB, 1, q.block[0]});
             }

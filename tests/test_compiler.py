@@ -354,6 +354,24 @@ def test_access_width_of_serial_order_rows(tmp_path):
         assert _vec(g.rmsnorm_quant(4096, cols), tmp_path) == few, cols
         assert _vec(g.rmsnorm_quant(4097, cols), tmp_path) == many, cols
     ir = g.with_dynamic_rows(g.safe_softmax(7919, 127), 7919)
-    assert _vec(ir, tmp_path, "hf_safe_softmax") == 1 and _vec(ir, tmp_path, "hf_safe_softmax_r4096") == 4
+    assert _vec(ir, tmp_path, "hf_safe_softmax") == 1 and _vec(ir, tmp_path, "hfa_safe_softmax_r4096") == 4
     # (int8 codes at a width below four: the exact pass stores them)
     assert hf.compile(g.rmsnorm_quant(5000, 127), options="").hsaco
+
+
+def test_kernels_by_row_count_keep_their_names_apart(tmp_path):
+    """Functions named like another function's kernel for some row counts
+    compile into one code object."""
+    g = hf.groups
+    body = lambda ir: ir[ir.index("{") + 1:ir.rindex("}")]
+    dyn = lambda ir, name: body(g.with_dynamic_rows(ir, 7919)).replace("@safe_softmax", "@" + name).replace("@w8a8_dequant", "@" + name)
+    sm, mm = g.safe_softmax(7919, 64), g.w8a8_dequant(7919, 64, 128)
+    ir = "module {" + dyn(sm, "sm") + dyn(sm, "sm_r256") + dyn(mm, "mm") + dyn(mm, "mm_16x16") + "}"
+    rc, err, prefix = emit(ir, tmp_path, options="dyn=runtime")
+    assert rc == 0, err
+    src = open(prefix + ".hip").read()
+    names = re.findall(r"__global__[^;{]*?\bvoid (\w+)\(", src)
+    alts = [ln.split()[1] for ln in open(prefix + ".manifest") if ln.startswith("alt ")]
+    assert len(names) == len(set(names)) and set(alts) <= set(names) and len(alts) >= 12
+    fns = re.findall(r"__device__[^;{]*? (\w+_(?:body|exact))\(", src)
+    assert len(fns) == len(set(fns))

@@ -188,10 +188,10 @@ def test_rmsq_f32_kernel_by_row_count():
     for cols, main, alts in ((1024, False, [("_wave", 2048, 256), ("_r4096", 4096, 1)]),
                              (2048, True, [("", 2048, 256), ("_r4096", 4096, 1), ("_r8192", 8192, 1)])):
         art = hf.compile(cat.get(f"rmsnorm_quant_f32_{cols}_rt"), options="dyn=runtime;emit=hip")
-        kern = art.blocks[0]["kernel"] if "kernel" in art.blocks[0] else "hf_rmsnorm_quant"
         got = [ln.split()[1:] for ln in open(art.manifest) if ln.startswith("alt ")]
         assert wave(art.blocks[0]) == main
-        assert [(a[0], int(a[1]), int(a[3])) for a in got] == [(kern + n, top, c) for n, top, c in alts]
+        assert [(a[0], int(a[1]), int(a[3])) for a in got] == [("hf_rmsnorm_quant" if not n else "hfa_rmsnorm_quant" + n, top, c)
+                                                                    for n, top, c in alts]
 
 
 @pytest.mark.gpu
