@@ -1350,11 +1350,12 @@ struct RowEmitter {
     else throw CompileError("row programs support rank-1 and rank-2 groups");
     if (!rowsHint) rowsHint = R;
     // vector width from the tensors that travel through HBM
-    int maxBytes = 1;
+    int maxBytes = 1, minBytes = 8;
     auto consider = [&](const Value *v) {
       if (!v->type.tensor || !A.map.count(v)) return;
       Sp s = spaceOfMap(A.map.at(v));
       if (s == Sp::Full || s == Sp::Col) maxBytes = std::max(maxBytes, elemBytes(v->type.elem));
+      if (s == Sp::Full) minBytes = std::min(minBytes, elemBytes(v->type.elem));
     };
     for (auto *a : A.f->args) consider(a);
     for (auto *r : A.f->returns) consider(r);
@@ -1388,9 +1389,23 @@ struct RowEmitter {
       RB = rowsHint <= 256 ? 1 : rowsHint <= 512 ? 2 : rowsHint <= 1024 ? 4 : 8;
       RPW = rowsHint <= 2048 ? 1 : rowsHint <= 4096 ? 2 : 4;
     } else {
-      // 128 bytes of a lane's row in flight (softmax, 4096 rows of 9544: 49.6
-      // -> 42.3 us against 64 bytes; 777 rows of 5003 8.5 -> 7.6)
-      const int64_t perLaneTarget = VEC * 8 < 32 ? VEC * 8 : 32;
+      // up to 32 elements of a lane's row in flight (128 bytes of f32; softmax,
+      // 4096 rows of 9544: 49.6 -> 42.3 us against 16 elements, 777 rows of 5003
+      // 8.5 -> 7.6).  16 of a narrow f32 row with one-byte results, whose lanes
+      // have more to do than to load (quantisation to int8, 300 rows of 4096: 4.2
+      // against 5.2 us, 16384 rows of 2048 27.6 against 30.4; to f32, 1000 rows of
+      // 3000: 5.2 and 4.5)
+      int64_t perLaneTarget = minBytes == 1 && C <= 4096 ? VEC * 4 : VEC * 8 < 32 ? VEC * 8 : 32;
+      // rows of 16-bit elements off 16-byte boundaries: few of them, or narrow
+      // ones, in the accesses that divide them and as many lanes (bf16 to fp8,
+      // dividing and full width: 64 rows of 2001 4.7 and 13.7 us, 1000 rows of 4095
+      // 17.4 and 19.2, 16384 rows of 603 41 and 49, but of 4095 212 and 163)
+      int div = VEC;
+      while (div > 1 && C % div) div /= 2;
+      if (VEC == 8 && div < VEC && (rowsHint <= 2048 || C <= 640)) {
+        VEC = div;
+        perLaneTarget = VEC * 4;
+      }
       int tr = 64;
       while (tr < 1024 && (int64_t)tr * perLaneTarget < C) tr *= 2;
       TR = tr;
@@ -4422,12 +4437,13 @@ std::vector<KernelPlan> lowerModule(Module &m, const LowerOptions &opt) {
         } else if (rows) {
           RowEmitter e(A, opt);
           p = e.run(kname, "LAST_AXIS_PBR");
-          // a launch-time row count: the serial-order schedules for fewer rows
-          if (A.rowsDyn && e.needOrdered)
-            for (int64_t rows : {256, 512, 1024, 2048, 4096}) {
+          // a launch-time row count: the schedules for fewer rows
+          if (A.rowsDyn)
+            for (int64_t rows : e.needOrdered ? std::vector<int64_t>{256, 512, 1024, 2048, 4096} : std::vector<int64_t>{2048}) {
               RowEmitter few(A, opt);
               few.rowsHint = rows;
               const KernelPlan q = few.run(altName(kname, "r" + std::to_string(rows)), "LAST_AXIS_PBR");
+              if (few.VEC == e.VEC && few.TR == e.TR && few.RB == e.RB && few.RPW == e.RPW) continue;
               p.source += q.source;
               p.alts.push_back({q.kernelName, rows, q.rowsB, 1, q.block[0]});
             }

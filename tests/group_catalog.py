@@ -1335,6 +1335,13 @@ def entries():
     e["cast_fp8"] = cast_fp8(4096)
     e["fp8_quant"] = fp8_quant(64, 4096)
     e["fp8_quant_ragged"] = fp8_quant(13, 1000)
+    # tree-reduced rows off 16-byte boundaries: several waves to a row, few and
+    # many rows (their access widths differ), and a launch-time row count
+    e["softmax_w5003"] = g.safe_softmax(37, 5003)
+    e["quant_i8_w5003"] = quant_i8_ties(37, 5003)
+    e["fp8_quant_w4999"] = fp8_quant(37, 4999)
+    e["fp8_quant_w2999_tall"] = fp8_quant(2100, 2999)
+    e["fp8_quant_w777_rt"] = g.with_dynamic_rows(fp8_quant(7919, 777), 7919)
     # un-fused host functions: the fusion front-end splits them into launch
     # programs of several groups
     e["prog_gemm_rmsnorm_quant"] = g.gemm_rmsnorm_quant(256, 512, 256)

@@ -375,3 +375,20 @@ def test_kernels_by_row_count_keep_their_names_apart(tmp_path):
     assert len(names) == len(set(names)) and set(alts) <= set(names) and len(alts) >= 12
     fns = re.findall(r"__device__[^;{]*? (\w+_(?:body|exact))\(", src)
     assert len(fns) == len(set(fns))
+
+
+def test_access_width_of_tree_reduced_rows(tmp_path):
+    """Rows of 16-bit elements off 16-byte boundaries take the dividing width
+    where they are few or narrow (a launch-time row count: a kernel for each),
+    f32 rows the full one; a narrow f32 row with one-byte results has more
+    lanes."""
+    g = hf.groups
+    for rows, cols, want in ((64, 2001, 1), (2048, 2001, 1), (2049, 2001, 8), (4096, 603, 1), (4096, 1500, 8), (64, 1500, 4),
+                             (64, 2000, 8), (4096, 640, 8)):
+        assert _vec(cat.fp8_quant(rows, cols), tmp_path) == want, (rows, cols)
+    ir = g.with_dynamic_rows(cat.fp8_quant(7919, 777), 7919)
+    assert _vec(ir, tmp_path, "hf_fp8_quant") == 8 and _vec(ir, tmp_path, "hfa_fp8_quant_r2048") == 1
+    assert _vec(g.safe_softmax(16, 5003), tmp_path) == 4
+    lanes = lambda ir, tmp: int(re.search(r"TR = (\d+)", open(emit(ir, tmp)[2] + ".hip").read()).group(1))
+    assert lanes(cat.quant_i8_ties(300, 4096), tmp_path) == 256 and lanes(cat.quant_i8_ties(300, 8192), tmp_path) == 256
+    assert lanes(g.safe_softmax(300, 8192), tmp_path) == 256

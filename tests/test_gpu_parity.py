@@ -417,6 +417,44 @@ def test_fp8_quant(gpu, name, rows, cols):
     assert np.array_equal(q, rq), f"{int((q != rq).sum())} fp8 codes differ"
 
 
+@pytest.mark.parametrize("name,rows,cols", [("fp8_quant_w4999", 37, 4999), ("fp8_quant_w2999_tall", 2100, 2999),
+                                            ("fp8_quant_w777_rt", 1, 777), ("fp8_quant_w777_rt", 2048, 777),
+                                            ("fp8_quant_w777_rt", 2049, 777)])
+def test_fp8_quant_off_16_bytes(gpu, name, rows, cols):
+    """Rows that start on any element, read in dividing and in full-width
+    accesses: bit-exact codes and scales."""
+    note(f"{name} {rows}x{cols}")
+    x = I.normal_bf16(I.SEED_BASE + 84, (rows, cols))
+    args = [x, zeros((rows, cols), np.uint8), zeros(rows, np.float32)]
+    q, s = run_gpu(name, args, gpu)
+    rq, rs = run_oracle(name, args)
+    assert np.array_equal(s.view(np.uint32), rs.view(np.uint32))
+    assert np.array_equal(q, rq), f"{int((q != rq).sum())} fp8 codes differ"
+
+
+def test_wide_rows_off_16_bytes(gpu):
+    """f32 rows of 5003 in a tree-reduced schedule of several waves a row: the
+    last row's end is the buffer's, and every byte around the results stays."""
+    import torch
+    note("softmax_w5003, quant_i8_w5003")
+    rng = np.random.default_rng(85)
+    x = rng.normal(0, 2, (37, 5003)).astype(np.float32)
+    out, = run_gpu("softmax_w5003", [x, zeros((37, 5003), np.uint16)], gpu)
+    ref, = run_oracle("softmax_w5003", [x, zeros((37, 5003), np.uint16)])
+    assert bf16_ulp_diff(out, ref).max() <= 1
+    grp = hf.compile(cat.get("softmax_w5003"), require_cached=True).load()
+    big = torch.full((37 * 5003 + 16,), 7.0, dtype=torch.bfloat16, device=gpu)
+    view = big[8:-8].view(37, 5003)
+    grp(torch.from_numpy(x).to(gpu), view)
+    torch.cuda.synchronize()
+    assert np.array_equal(view.view(torch.int16).cpu().numpy().view(np.uint16), out)
+    assert bool((big[:8] == 7).all()) and bool((big[-8:] == 7).all())
+    args = [x, rng.uniform(0.01, 0.1, 37).astype(np.float32), zeros((37, 5003), np.int8), zeros(37, np.float32)]
+    got, ref = run_gpu("quant_i8_w5003", args, gpu), run_oracle("quant_i8_w5003", args)
+    for a, b in zip(got, ref):
+        assert np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8))
+
+
 # ------------------------------------------------------------------ generic lowering
 def test_eltwise_mix(gpu):
     note("eltwise_mix")
