@@ -40,7 +40,8 @@
  *   ordered_fp_sums=0|1     serial-order fp32 sums for every linalg.reduce addf
  *   rmsq_kernel=0|1         RMSNorm + dynamic int8 quantisation groups: 1 (the
  *                           default) through the one-wave-per-row exact
- *                           parallel sum where the widths allow, 0 through the
+ *                           parallel sum where the widths (of an f32 x: and
+ *                           the row count) make it the faster, 0 through the
  *                           generic row program
  *   rmsn_kernel=1           the same groups through the chain-wave kernel
  *   mx_exact=1              fp8 hfusion.matmul_mx through scaled bf16 operands
