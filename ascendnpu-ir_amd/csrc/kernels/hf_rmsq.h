@@ -252,31 +252,34 @@ __device__ __forceinline__ void rmsq_rows(const XT *__restrict__ x, const uint16
     const uint32_t G = NG * lane0 + g;
     rdPtr[g] = lds + (G ^ ((G >> 4) & MASK));
   }
-  // an f32 x may start on any element (a view into a larger buffer), the
-  // 16-byte DMA only on its own size
-  const bool aligned16 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)x & 15u) == 0;
-  auto issueRow = [&](int64_t r) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's reads of the buffer are done
-    const char *rowp = reinterpret_cast<const char *>(x + uniform_i64(r) * C);
-    if (!BF && !aligned16) {
-      // the same layout in 4-byte pieces: instruction k fills slots 16k ..
-      // 16k + 15 (at most 32 in flight: the wave's counter holds 63)
-#pragma unroll 1
-      for (int k = 0; k < 4 * NG; ++k) {
-        const uint32_t off = 16u * (((uint32_t)lane0 / 4) ^ ((uint32_t)k & MASK)) + 4u * ((uint32_t)lane0 % 4);
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(rowp + 256 * k),
-                     "s"(__builtin_amdgcn_readfirstlane(ldsBase + 256u * k))
-                     : "memory");
-        if (k % 32 == 31) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      return;
-    }
+  // 16 bytes a lane; an f32 x may start on any element (a view into a larger
+  // buffer), and from other than 16-byte addresses its rows are moved in 4-byte
+  // pieces into the same layout: instruction k fills slots 16k .. 16k + 15 (at
+  // most 32 in flight: the wave's counter holds 63)
+  auto issueRow16 = [&](const char *rowp) {
 #pragma unroll
     for (int k = 0; k < NG; ++k) {
       asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(dmaOff[k & (MASK / 4)]),
-                   "s"(rowp + 1024 * k), "s"(__builtin_amdgcn_readfirstlane(ldsBase + 1024u * k))
+                   "s"(rowp + 1024 * k), "s"(BF ? ldsBase + 1024u * k : __builtin_amdgcn_readfirstlane(ldsBase + 1024u * k))
                    : "memory");
     }
+  };
+  auto issueRow4 = [&](const char *rowp) {
+#pragma unroll 1
+    for (int k = 0; k < 4 * NG; ++k) {
+      const uint32_t off = 16u * (((uint32_t)lane0 / 4) ^ ((uint32_t)k & MASK)) + 4u * ((uint32_t)lane0 % 4);
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(rowp + 256 * k),
+                   "s"(__builtin_amdgcn_readfirstlane(ldsBase + 256u * k))
+                   : "memory");
+      if (k % 32 == 31) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+  };
+  auto issueRow = [&](int64_t r) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's reads of the buffer are done
+    const char *rowp = reinterpret_cast<const char *>(x + uniform_i64(r) * C);
+    if constexpr (BF) issueRow16(rowp);
+    else if (__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)x & 15u) == 0) issueRow16(rowp);
+    else issueRow4(rowp);
   };
   // staggered start: the second wave on each SIMD (w / 4 = 1) issues its
   // first row C/2 cycles late and the third (which has one row fewer) 2C
