@@ -1399,10 +1399,11 @@ struct RowEmitter {
       // rows of 16-bit elements off 16-byte boundaries: few of them, or narrow
       // ones, in the accesses that divide them and as many lanes (bf16 to fp8,
       // dividing and full width: 64 rows of 2001 4.7 and 13.7 us, 1000 rows of 4095
-      // 17.4 and 19.2, 16384 rows of 603 41 and 49, but of 4095 212 and 163)
+      // 17.4 and 19.2, 16384 rows of 603 41 and 49, but of 4095 212 and 163); the
+      // narrowest of any type (f32 quantisation, 16384 rows of 127: 6.0 and 6.9)
       int div = VEC;
       while (div > 1 && C % div) div /= 2;
-      if (VEC == 8 && div < VEC && (rowsHint <= 2048 || C <= 640)) {
+      if (div < VEC && (C <= 160 || (VEC == 8 && (rowsHint <= 2048 || C <= 640)))) {
         VEC = div;
         perLaneTarget = VEC * 4;
       }

@@ -389,6 +389,8 @@ def test_access_width_of_tree_reduced_rows(tmp_path):
     ir = g.with_dynamic_rows(cat.fp8_quant(7919, 777), 7919)
     assert _vec(ir, tmp_path, "hf_fp8_quant") == 8 and _vec(ir, tmp_path, "hfa_fp8_quant_r2048") == 1
     assert _vec(g.safe_softmax(16, 5003), tmp_path) == 4
+    for cols, want in ((127, 1), (130, 2), (160, 4), (161, 4)):
+        assert _vec(cat.quant_ties(16384, cols), tmp_path) == want, cols
     lanes = lambda ir, tmp: int(re.search(r"TR = (\d+)", open(emit(ir, tmp)[2] + ".hip").read()).group(1))
     assert lanes(cat.quant_i8_ties(300, 4096), tmp_path) == 256 and lanes(cat.quant_i8_ties(300, 8192), tmp_path) == 256
     assert lanes(g.safe_softmax(300, 8192), tmp_path) == 256
